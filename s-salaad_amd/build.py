@@ -10,6 +10,9 @@ With --checked, the same sources are built with SSL_DEVICE_CHECKS=1 into
 read from plans and records and report a bad one in the call's status word
 (ssl_device_checks). Load it with SSALAAD_AMD_LIB=<its path>.
 
+The host call path csrc_py/hostcall.c is built with the C compiler into
+`ssalaad_amd/hostcall.<abi>.so`, a CPython extension that links to neither.
+
 Usage: python s-salaad_amd/build.py [-v] [--checked]
 """
 
@@ -19,6 +22,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 import time
 from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
@@ -76,7 +80,26 @@ COMMON_FLAGS = [
 ]
 
 
+def build_hostcall(verbose: bool = False) -> Path:
+    cc = shutil.which("gcc") or shutil.which("cc") or shutil.which("clang")
+    if cc is None:
+        raise RuntimeError("no C compiler found; the host call path cannot be built")
+    out = HERE / "ssalaad_amd" / ("hostcall" + sysconfig.get_config_var("EXT_SUFFIX"))
+    tmp = out.with_name(out.name + ".tmp")
+    cmd = [cc, "-O2", "-std=c11", "-shared", "-fPIC", "-Wall", "-I", str(HERE.parent / "include"),
+           "-I", sysconfig.get_paths()["include"], str(HERE / "csrc_py" / "hostcall.c"),
+           "-o", str(tmp)]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"building the host call path failed:\n{res.stderr}")
+    os.replace(tmp, out)
+    if verbose:
+        print(f"[build] wrote {out}")
+    return out
+
+
 def build(verbose: bool = False, jobs: int = 8, checked: bool = False) -> Path:
+    build_hostcall(verbose)
     hipcc = _hipcc()
     out = OUT_CHECKED if checked else OUT
     build_dir = BUILD_DIR / "checked" if checked else BUILD_DIR

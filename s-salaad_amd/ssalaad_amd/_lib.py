@@ -225,6 +225,36 @@ def load() -> ctypes.CDLL:
     return lib
 
 
+_hostcall = None
+
+
+def hostcall():
+    """The compiled host call path (once); raises if it was not built."""
+    global _hostcall
+    if _hostcall is None:
+        try:
+            from . import hostcall as mod
+        except ImportError as e:
+            raise RuntimeError(
+                "the host call path is not built; run `python s-salaad_amd/build.py` "
+                "(or __graft_entry__.build()) first") from e
+        if mod.MEMBER_BYTES != ctypes.sizeof(SlrMember):
+            raise RuntimeError("hostcall was built against another ssalaad_amd.h; build again")
+        _hostcall = mod
+    return _hostcall
+
+
+_ADDRESS: dict[str, int] = {}
+
+
+def entry_address(name: str) -> int:
+    """The address of an exported entry point."""
+    a = _ADDRESS.get(name)
+    if a is None:
+        a = _ADDRESS[name] = ctypes.cast(getattr(load(), name), ctypes.c_void_p).value
+    return a
+
+
 def _check_single_hip_runtime() -> None:
     """Two HIP runtimes in one process would split device state; refuse that."""
     try:

@@ -265,6 +265,7 @@ class DevicePlan:
         if self._exchange is None or self._exchange.numel() < nbytes:
             if self._exchange is not None:
                 self._retired.append(self._exchange)
+            _replaced()
             self._exchange = torch.zeros(max(int(nbytes), 256), dtype=torch.uint8,
                                          device=self.table.device)
         return self._exchange
@@ -277,6 +278,20 @@ class DevicePlan:
         if self._exchange is None:
             return 0
         return int(self._exchange[:8].view(torch.int64)[0].item())
+
+
+# Counts every replacement of a pool buffer or exchange area: a call bound to
+# them at one value is bound to the live ones while the value stands.
+_generation = 0
+
+
+def generation() -> int:
+    return _generation
+
+
+def _replaced() -> None:
+    global _generation
+    _generation += 1
 
 
 _WORKSPACES: dict[tuple[int, int], torch.Tensor] = {}
@@ -298,6 +313,7 @@ def _grown(pool, key, n, dtype, device, minimum):
         if buf is not None:
             size = max(size, 2 * buf.numel())
             _RETIRED.append(buf)
+        _replaced()
         buf = torch.zeros(size, dtype=dtype, device=device)
         pool[key] = buf
     return buf

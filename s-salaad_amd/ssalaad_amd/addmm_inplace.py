@@ -51,7 +51,7 @@ def get_tuned_config(block_p: int, block_q: int) -> dict:
 
 
 class _StructPlan:
-    __slots__ = ("versions", "col_ref", "act_ref", "plans", "NB_K")
+    __slots__ = ("versions", "col_ref", "act_ref", "plans", "NB_K", "calls")
 
     def __init__(self, versions, col, act, NB_K):
         self.versions = versions
@@ -59,6 +59,8 @@ class _StructPlan:
         self.act_ref = weakref.ref(act)
         self.plans: dict[int, _runtime.DevicePlan] = {}
         self.NB_K = NB_K
+        # streaming calls already made: (shapes, stream) -> (generation, launcher)
+        self.calls: dict[tuple, tuple] = {}
 
 
 _PLAN_ATTR = "_ssl_struct_plan"
@@ -181,6 +183,33 @@ def _aligned_rows(t: torch.Tensor) -> bool:
     return t.stride(-1) == 1 and t.data_ptr() % 16 == 0 and (t.stride(0) * eb) % 16 == 0
 
 
+_MAX_CALLS = 16  # kept launchers per structure
+
+
+def _repeat(out, x, crow, col, values, active) -> bool:
+    """Issue a call that repeats an earlier streaming call's structure and
+    shapes on its stream, with contiguous 16-byte aligned tensors; False when
+    it is not one (or would be refused): the full path then handles it."""
+    sp = getattr(crow, _PLAN_ATTR, None)
+    if sp is None or sp.col_ref() is not col or sp.act_ref() is not active:
+        return False
+    dev = crow.device
+    if torch._C._cuda_getDevice() != dev.index:
+        return False
+    hit = sp.calls.get((out.shape, x.shape, values.shape, values.dtype,
+                        torch._C._cuda_getCurrentRawStream(dev.index)))
+    if hit is None or hit[0] != _runtime.generation():
+        return False
+    if (out.dtype is not values.dtype or x.dtype is not values.dtype or out.device != dev
+            or x.device != dev or values.device != dev
+            or not (out.is_contiguous() and x.is_contiguous() and values.is_contiguous())
+            or sp.versions[:5] != (crow._version, col._version, active._version, col.data_ptr(),
+                                   active.data_ptr())):
+        return False
+    o, xp, v = out.data_ptr(), x.data_ptr(), values.data_ptr()
+    return (o | xp | v) % 16 == 0 and hit[1].launch(o, xp, v) == 0
+
+
 def bsr_addmm_inplace_(
     out_inplace: torch.Tensor,
     x: torch.Tensor,
@@ -190,6 +219,8 @@ def bsr_addmm_inplace_(
     active_rows: torch.Tensor,
 ) -> None:
     """In place ``out_inplace += x @ S.T`` on the active block-rows of S."""
+    if _repeat(out_inplace, x, crow_indices, col_indices, values, active_rows):
+        return
     if out_inplace.dtype not in _TORCH_DTYPES:
         raise TypeError(
             f"HIP BSR kernel supports float16/bfloat16/float32, got {out_inplace.dtype}"
@@ -275,6 +306,18 @@ def bsr_addmm_inplace_(
             _lib.stream_ptr(dev),
         )
     _lib.check(rc, "ssl_bsr_addmm_inplace")
+    if (pf is None and target is out_inplace and out_inplace.is_contiguous()
+            and x.is_contiguous() and col is col_indices and dev.index is not None):
+        sp = getattr(crow_indices, _PLAN_ATTR)
+        if len(sp.calls) >= _MAX_CALLS:
+            sp.calls.clear()
+        sp.calls[(out_inplace.shape, x.shape, values.shape, values.dtype, _lib.stream_ptr(dev))] = (
+            _runtime.generation(),
+            _lib.hostcall().OpCall(
+                _lib.entry_address("ssl_bsr_addmm_inplace"), _runtime.status_word(dev).host_ptr,
+                N, K, col.data_ptr(), vals.shape[0], plan.table.data_ptr(), plan.n_chunks,
+                plan.n_slots, M, N, K, NB, block_p, block_q, dt, cnt.data_ptr(), cnt.numel(),
+                ws.data_ptr(), ws.numel(), _lib.stream_ptr(dev)))
     if target is not out_inplace:
         out_inplace.copy_(target)
 

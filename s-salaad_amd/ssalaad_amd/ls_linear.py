@@ -31,6 +31,7 @@ Differences from the reference, all extensions:
 
 from __future__ import annotations
 
+import ctypes
 import weakref
 
 import numpy as np
@@ -64,8 +65,11 @@ class _KernelState:
                  block: tuple[int, int] | None = None):
         dtype = mod.A.dtype
         self.key = mod._weights_key()
+        self.watch = _lib.hostcall().Watch(mod._buffers)  # the same, compared on each call
         self.device = device
+        self.dtype = dtype
         self.dtype_code = _lib.dtype_code(dtype)
+        self.index = device.index if device.index is not None else torch.cuda.current_device()
         self.elem = torch.empty((), dtype=dtype).element_size()
         n, m, r = mod.out_features, mod.in_features, mod.r
         p, q = block if block is not None else mod._kernel_block
@@ -115,9 +119,14 @@ class _KernelState:
         # kernel block-columns: a stored block-column of bq features is bq / q of them
         bq = getattr(mod, "block_q", None) or q
         self.NBK = -(-m // bq) * (bq // q)
+        # contiguous x rows are 16-byte aligned
+        self._x_aligned = m > 0 and (m * self.elem) % 16 == 0
         self._plans: dict[int, _runtime.DevicePlan] = {}
         # fused calls led by this state: (M, stream, linears) -> _LaunchCall
-        self._calls: dict[tuple, "_LaunchCall"] = {}
+        self._calls: dict[tuple, "_Descriptors"] = {}
+        # the same by the linears as called (before prefill_view), with the
+        # launcher that issues them
+        self._launchers: dict[tuple, tuple] = {}
         self._pf_plans: dict[int, _runtime.DevicePrefillPlan] = {}
         self._values_pq: torch.Tensor | None = None
 
@@ -352,6 +361,37 @@ _MAX_CALLS = 16  # cached launch descriptors per leading state
 _PREFILL_MIN_ROWS = 128  # ssl_prefill_min_rows(): fewer token rows always stream
 
 
+def _relaunch(states, x: torch.Tensor, out_features):
+    """A fused call whose descriptors are kept, with contiguous aligned x: the
+    outputs, or None when the call is not one of those (or would be refused),
+    which `_launch` then handles."""
+    st0 = states[0]
+    if not (st0._x_aligned and x.is_contiguous()):
+        return None
+    xp = x.data_ptr()
+    shape = x.shape
+    M = shape[0] if len(shape) == 2 else x.numel() // st0.m
+    key = (M, torch._C._cuda_getCurrentRawStream(st0.index), *map(id, states))
+    hit = st0._launchers.get(key)
+    if hit is None or xp % 16 or hit[0] != _runtime.generation():
+        return None
+    _, _, launcher, called, pads = hit  # `called` is held, so its ids are not reused
+    for a, b in zip(called, states):
+        if a is not b:
+            return None
+    lead = shape[:-1]
+    if len(pads) == 1:
+        n, pad = out_features[0], pads[0]
+        y = torch.empty((*lead, pad), dtype=x.dtype, device=x.device)
+        if launcher.launch(xp, y.data_ptr()) != 0:
+            return None
+        return (y if n == pad else y[..., :n],)
+    ys = [torch.empty((*lead, pad), dtype=x.dtype, device=x.device) for pad in pads]
+    if launcher.launch(xp, *[y.data_ptr() for y in ys]) != 0:
+        return None
+    return [y if n == pad else y[..., :n] for y, n, pad in zip(ys, out_features, pads)]
+
+
 def _launch(states: list["_KernelState"], x: torch.Tensor, out_features: list[int]):
     """One fused launch computing every state's linear of the same x.
 
@@ -363,6 +403,7 @@ def _launch(states: list["_KernelState"], x: torch.Tensor, out_features: list[in
     _runtime.check_status(dev)
     st0 = states[0]
     orig = x.shape
+    called = states
     x2 = st0.rows(x)
     M = x2.shape[0]
     if M >= _PREFILL_MIN_ROWS:
@@ -379,20 +420,35 @@ def _launch(states: list["_KernelState"], x: torch.Tensor, out_features: list[in
         stream = _lib.stream_ptr(dev)
         key = (M, stream, tuple(map(id, states)))
         d = st0._calls.get(key)  # its states are held, so their ids are not reused
+        again = d is not None
         if d is None or any(a is not b for a, b in zip(d.states, states)):
             G = 0
             rows = sum(st.NB for st in states)
             if st0.takes_prefill(M, rows):
                 G = int(lib.ssl_prefill_group(M, rows, st0.p, st0.q))
+            again = False
             if len(st0._calls) >= _MAX_CALLS:
                 st0._calls.clear()
             d = st0._calls[key] = _Descriptors(states, M, G)
+        generation = _runtime.generation()
         d.bind(dev)
         for mb, y in zip(d.members, ys):
             mb.y = y.data_ptr()
         rc = lib.ssl_slr_forward_group(x2.data_ptr(), x2.stride(0), M, st0.m, st0.m_pad, st0.p,
                                        st0.q, st0.dtype_code, d.members, len(states), stream)
         _lib.check(rc, "ssl_slr_forward_group")
+        if again and called[0]._x_aligned and generation == _runtime.generation():
+            # from the third call of this token count, stream and linears on,
+            # aligned contiguous x goes straight to the launcher
+            launcher = _lib.hostcall().GroupCall(
+                _lib.entry_address("ssl_slr_forward_group"), _runtime.status_word(dev).host_ptr,
+                st0.m, M, st0.m, st0.m_pad, st0.p, st0.q, st0.dtype_code,
+                ctypes.addressof(d.members), len(states), stream)
+            kept = called[0]._launchers
+            if len(kept) >= _MAX_CALLS:
+                kept.clear()
+            kept[(M, stream, *map(id, called))] = (
+                generation, d, launcher, tuple(called), tuple(st.n_pad for st in states))
     return _outputs(states, ys, out_features, orig[:-1])
 
 
@@ -466,6 +522,12 @@ class _LRSLinearBase(nn.Module):
         return st
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
+        st = self._state
+        if (st is not None and x.dtype is st.dtype and x.shape[-1] == self.in_features
+                and x.device == st.device and st.watch.unchanged(self._buffers)):
+            out = _relaunch((st,), x, (self.out_features,))
+            if out is not None:
+                return out[0]
         if x.dtype != self.A.dtype:
             raise TypeError(f"input dtype {x.dtype} does not match the weights' {self.A.dtype}")
         if x.shape[-1] != self.in_features:
@@ -675,7 +737,27 @@ class LRSLinearGroup(nn.Module):
         self.members = nn.ModuleList(linears)
         self.in_features = first.in_features
 
+    def _again(self, x: torch.Tensor):
+        """The outputs of a call that repeats an earlier one's shape with every
+        member's weights unchanged, else None."""
+        states, outf = [], []
+        for mod in self.members._modules.values():
+            st = mod._state
+            if st is None or not st.watch.unchanged(mod._buffers):
+                return None
+            states.append(st)
+            outf.append(mod.out_features)
+        st0 = states[0]
+        if (x.dtype is not st0.dtype or x.shape[-1] != self.in_features
+                or x.device != st0.device):
+            return None
+        out = _relaunch(states, x, outf)
+        return None if out is None else tuple(out)
+
     def forward(self, x: torch.Tensor) -> tuple[torch.Tensor, ...]:
+        out = self._again(x)
+        if out is not None:
+            return out
         first = self.members[0]
         if x.dtype != first.A.dtype:
             raise TypeError(f"input dtype {x.dtype} does not match the weights' {first.A.dtype}")

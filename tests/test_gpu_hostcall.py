@@ -1,0 +1,152 @@
+"""The kept launchers of eager calls (hostcall): a repeated call equals the first
+one, and whatever differs from it — weights, shapes, strides, streams, a refused
+status — takes the full path again with the full path's results and errors."""
+
+import pytest
+import torch
+
+from ssalaad_amd import LRSLinear, LRSLinearGroup, _lib, _runtime, clear_wait_status
+
+pytestmark = pytest.mark.gpu
+
+
+def _linear(seed, n=192, m=160, r=24, p=32, dtype=torch.bfloat16, bias=True):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    rnd = lambda *s: (torch.randn(*s, generator=g, device="cuda") * 0.1).to(dtype)  # noqa: E731
+    nb, nbk = -(-n // p), -(-m // p)
+    S = rnd(nb * p, nbk * p)
+    S[n:], S[:, m:] = 0, 0
+    keep = torch.rand(nb, 1, nbk, 1, generator=g, device="cuda") < 0.6
+    S = (S.view(nb, p, nbk, p) * keep).view(nb * p, nbk * p)
+    mod = LRSLinear(rnd(n, r), rnd(r, m), S.to_sparse_bsr((p, p)), in_features=m, out_features=n,
+                    bias=rnd(n) if bias else None, block_p=p, block_q=p)
+    return mod, S[:n, :m]
+
+
+def _expect(mod, S, x):
+    y = (x.double() @ mod.B.double().T) @ mod.A.double().T + x.double() @ S.double().T
+    return y if mod.bias is None else y + mod.bias.double()
+
+
+def _close(y, ref):
+    # t and y are each rounded once to the 16-bit dtype (2^-9): at most 1e-2 of the largest value
+    assert float((y.double() - ref).abs().max()) <= 1e-2 * float(ref.abs().max())
+
+
+@pytest.mark.parametrize("n,m,tokens", [(192, 160, 1), (150, 160, 5), (192, 150, 16), (64, 32, 129),
+                                        (192, 160, 200)])
+def test_repeated_linear_calls(n, m, tokens, gpu_device):
+    mod, S = _linear(0, n, m)
+    x = torch.randn(tokens, m, device="cuda").to(torch.bfloat16)
+    first = mod(x).clone()
+    _close(first, _expect(mod, S, x))
+    for _ in range(3):
+        assert torch.equal(mod(x), first)
+    x2 = torch.randn_like(x)
+    _close(mod(x2), _expect(mod, S, x2))
+    # leading dimensions, a row-strided x, an unaligned x
+    assert torch.equal(mod(x.view(tokens, 1, m)), first.view(tokens, 1, n))
+    if tokens == 1:
+        assert mod(x[0]).shape == (n,) and torch.equal(mod(x[0]), first[0])
+    wide = torch.empty(tokens, m + 24, device="cuda", dtype=x.dtype)
+    wide[:, 3:m + 3] = x
+    assert torch.equal(mod(wide[:, 3:m + 3]), first)
+    assert mod(x[:0]).shape == (0, n)
+
+
+def test_changed_weights_and_refusals(gpu_device):
+    mod, S = _linear(1)
+    x = torch.randn(4, 160, device="cuda").to(torch.bfloat16)
+    mod(x), mod(x)
+    mod.A.mul_(2)                       # in place
+    _close(mod(x), _expect(mod, S, x))
+    mod.B = mod.B * 3                   # replaced
+    _close(mod(x), _expect(mod, S, x))
+    mod.bias.data = mod.bias * 0 + 1    # new storage, same tensor object
+    _close(mod(x), _expect(mod, S, x))
+    mod.bias = None
+    _close(mod(x), _expect(mod, S, x))
+    with pytest.raises(TypeError):
+        mod(x.half())
+    with pytest.raises(ValueError):
+        mod(x[:, :128])
+    with pytest.raises(ValueError):
+        mod(x.cpu())
+    word = _runtime.status_word(x.device)
+    word._word.value = 1
+    try:
+        with pytest.raises(RuntimeError):
+            mod(x)
+    finally:
+        clear_wait_status()
+    _close(mod(x), _expect(mod, S, x))
+    mod.half()
+    _close(mod(x.half()), _expect(mod, S, x.half()))
+
+
+def test_groups_streams_and_grown_pools(gpu_device):
+    a, Sa = _linear(2, bias=False)
+    b, Sb = _linear(3, n=96)
+    grp = LRSLinearGroup(a, b)
+    x = torch.randn(3, 160, device="cuda").to(torch.bfloat16)
+    first = [y.clone() for y in grp(x)]
+    for y, (mod, S) in zip(first, ((a, Sa), (b, Sb))):
+        _close(y, _expect(mod, S, x))
+    assert all(torch.equal(u, v) for u, v in zip(grp(x), first))
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        for _ in range(2):
+            assert all(torch.equal(u, v) for u, v in zip(grp(x), first))
+    side.synchronize()
+    before = _runtime.generation()
+    big = torch.randn(400, 160, device="cuda").to(torch.bfloat16)  # a larger exchange area
+    grp(big)
+    assert _runtime.generation() > before
+    for _ in range(2):
+        assert all(torch.equal(u, v) for u, v in zip(grp(x), first))
+    b.A.add_(1)
+    _close(grp(x)[1], _expect(b, Sb, x))
+
+
+@pytest.mark.parametrize("tokens", [1, 7, 100])
+def test_repeated_op_calls(tokens, gpu_device):
+    mod, S = _linear(4, bias=False)
+    crow, col, vals = mod.S_crow, mod.S_col, mod.S_values
+    act = mod.S_active_rows
+    op = torch.ops.ssalaad.tilelang_bsr_addmm_inplace_dense_
+    x = torch.randn(tokens, 160, device="cuda").to(torch.bfloat16)
+    out0 = torch.randn(tokens, 192, device="cuda").to(torch.bfloat16)
+
+    def run(x_, out_, v_):
+        out_ = out_.clone()
+        op(out_, x_, crow, col, v_, act)
+        return out_
+
+    first = run(x, out0, vals)
+    _close(first, out0.double() + x.double() @ S.double().T)
+    for _ in range(2):
+        assert torch.equal(run(x, out0, vals), first)
+    _close(run(x, out0, vals * 2), out0.double() + 2 * (x.double() @ S.double().T))
+    vals.mul_(0.5)
+    _close(run(x, out0, vals), out0.double() + 0.5 * (x.double() @ S.double().T))
+    vals.mul_(2)
+    wide = torch.empty(tokens, 168, device="cuda", dtype=x.dtype)
+    wide[:, 1:161] = x
+    assert torch.equal(run(wide[:, 1:161], out0, vals), first)
+    with pytest.raises(TypeError):
+        run(x.half(), out0, vals)
+    act2 = act[:-1].clone()  # fewer active rows: the last block-row keeps its bits
+    out = out0.clone()
+    op(out, x, crow, col, vals, act2)
+    assert torch.equal(out[:, -32:], out0[:, -32:]) and torch.equal(out[:, :-32], first[:, :-32])
+
+
+def test_launchers_check_their_arguments():
+    h = _lib.hostcall()
+    with pytest.raises(ValueError):
+        h.GroupCall(0, 0, 1, 1, 1, 64, 16, 16, 1, 0, 1, 0)
+    with pytest.raises(ValueError):
+        h.OpCall(0, 0, *[0] * 19)
+    w = h.Watch({"a": torch.zeros(2), "b": None})
+    assert not w.unchanged({"a": torch.zeros(2)})
