@@ -84,13 +84,13 @@ int ssl_status_word_alloc(void** host_ptr, void** device_ptr);
  *   SSL_DEBUG_WAIT_UNREACHABLE  nonzero: every wait of the fused kernel targets
  *                               a count no launch reaches, so each gives up
  *                               after its polls and reports it.
- *   SSL_DEBUG_PREFILL_SPLIT     0: the library decides whether a fused
- *                               prefill call splits its row groups' sparse
- *                               steps (and its latent's in_features) across
- *                               workgroups; 1: never; 2 to 4: every fused
- *                               prefill call splits its row groups in that
- *                               many parts (when the caller's workspace holds
- *                               the partial tiles).
+ *   SSL_DEBUG_PREFILL_SPLIT     0: the library decides whether a prefill call
+ *                               (the fused linear's or the op's) splits its row
+ *                               groups' sparse steps (and its latent's
+ *                               in_features) across workgroups; 1: never; 2
+ *                               to 4: every such call splits its row groups in
+ *                               that many parts (when the caller's workspace
+ *                               holds the partial tiles).
  *   SSL_DEBUG_CHAIN_FRAG        0: the library decides whether a chained launch
  *                               of 32- or 64-wide blocks passes its stages'
  *                               inputs in fragment order (ssl_slr_stage.xf);
@@ -247,6 +247,9 @@ int32_t ssl_slr_takes_prefill(int64_t M, int64_t n_rows, int32_t block_p, int32_
  * ------------------------------------------------------------------------- */
 int32_t ssl_bsr_addmm_takes_prefill(int64_t M, int64_t n_rows, int32_t block_p,
                                     int32_t block_q, int32_t dtype);
+/* The sizes include what a prefill call's K parts take; a call given less (at
+ * least the streaming kernel's counters and partial tiles of split rows) runs
+ * whole row groups. */
 int64_t ssl_bsr_addmm_workspace_size(int64_t M, int64_t NB, int32_t block_p,
                                      int64_t n_slots);
 int64_t ssl_bsr_addmm_counter_count(int64_t M, int64_t NB);

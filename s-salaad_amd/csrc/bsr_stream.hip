@@ -138,6 +138,23 @@ Layout slr_layout(int64_t M, int64_t NB, int p, int64_t r_pad, int64_t m_pad, in
   return L;
 }
 
+// The in-place op's scratch: the streaming kernel's row counters and partial
+// tiles (what a call cannot do without), and the bytes the tiled kernel's K
+// parts may take besides.
+int64_t op_counters_min(int64_t M, int64_t NB) {
+  const int MT = tile_mt(M);
+  return (M + 16 * MT - 1) / (16 * MT) * NB;
+}
+int64_t op_workspace_min(int64_t M, int32_t block_p, int64_t n_slots) {
+  const int MT = tile_mt(M);
+  const int64_t MG = (M + 16 * MT - 1) / (16 * MT);
+  return align_up(4 * MG * n_slots * (16 * MT * block_p), 256);
+}
+int64_t op_split_bytes(int64_t M, int64_t NB, int32_t block_p) {
+  if (M < kPrefillMinM || !prefill_block(block_p, block_p, SSL_BF16)) return 0;
+  return prefill_split_bytes(M, NB, block_p, 0, 0, SSL_BF16, device_cus());
+}
+
 // K chunks of this launch's latent: as many as the free compute units allow
 // (latent workgroups — per_chunk of them per K chunk — and the n_stream row
 // workgroups all resident at once), at most n_kc_max; then evened out so no
@@ -519,17 +536,16 @@ int32_t ssl_bsr_addmm_takes_prefill(int64_t M, int64_t n_rows, int32_t block_p, 
   return 1;
 }
 
+// Row counters, then (many token rows) one arrival word per (64-row token
+// tile, block-row) for the tiled kernel's K parts, all zero at rest.
 int64_t ssl_bsr_addmm_counter_count(int64_t M, int64_t NB) {
-  const int MT = tile_mt(M);
-  const int64_t MG = (M + 16 * MT - 1) / (16 * MT);
-  return MG * NB;
+  return op_counters_min(M, NB) + (M >= kPrefillMinM ? (M + 63) / 64 * NB : 0);
 }
 
+// The streaming kernel's partial tiles of split rows, then (many token rows)
+// the tiled kernel's partial tiles of its K parts.
 int64_t ssl_bsr_addmm_workspace_size(int64_t M, int64_t NB, int32_t block_p, int64_t n_slots) {
-  (void)NB;
-  const int MT = tile_mt(M);
-  const int64_t MG = (M + 16 * MT - 1) / (16 * MT);
-  return align_up(4 * MG * n_slots * (16 * MT * block_p), 256);
+  return op_workspace_min(M, block_p, n_slots) + align_up(op_split_bytes(M, NB, block_p), 256);
 }
 
 int ssl_bsr_addmm_inplace(void* out, int64_t ldo, const void* x, int64_t ldx, const int32_t* col,
@@ -560,14 +576,13 @@ int ssl_bsr_addmm_inplace(void* out, int64_t ldo, const void* x, int64_t ldx, co
   if (!aligned(x, 16) || (ldx * eb) % 16 || !aligned(values, 16))
     return fail(SSL_ERR_INVALID, "x rows and values must be 16-byte aligned");
   if (!aligned(out, 16) || (ldo * eb) % 16) return fail(SSL_ERR_INVALID, "out rows must be 16-byte aligned");
-  const int64_t need = ssl_bsr_addmm_workspace_size(M, NB, block_p, n_slots);
+  const int64_t need = op_workspace_min(M, block_p, n_slots);
   if (workspace_bytes < need || (need > 0 && !workspace))
     return fail(SSL_ERR_WORKSPACE, "workspace of %lld bytes needed", (long long)need);
   if (workspace && !aligned(workspace, 256))
     return fail(SSL_ERR_WORKSPACE, "workspace must be 256-byte aligned");
-  if (n_counters < ssl_bsr_addmm_counter_count(M, NB) || !counters)
-    return fail(SSL_ERR_WORKSPACE, "%lld zeroed counters needed",
-                (long long)ssl_bsr_addmm_counter_count(M, NB));
+  if (n_counters < op_counters_min(M, NB) || !counters)
+    return fail(SSL_ERR_WORKSPACE, "%lld zeroed counters needed", (long long)op_counters_min(M, NB));
 
   if (nnz < 0 || !slab_count_ok(nnz, block_q / (4 * stream_ke(dtype, block_q))))
     return fail(SSL_ERR_UNSUPPORTED, "too many blocks (%lld) for one call", (long long)nnz);
@@ -591,11 +606,25 @@ int ssl_bsr_addmm_inplace(void* out, int64_t ldo, const void* x, int64_t ldx, co
     pm.y = out; pm.ldy = ldo; pm.values_pq = values_pq; pm.NB = (int)NB;
     pm.values_bytes = nnz * block_p * block_q * eb;
     pm.groups = pf_groups; pm.steps = pf_steps; pm.n_groups = (int)pf_n_groups;
-    pm.ksplit = 1;  // the op's row kernel runs whole row groups
     rows.bm = prefill_row_tile(M, n_chunks, pf_group, block_p, device_cus(), dtype, 0);
     const int64_t T = (M + rows.bm - 1) / rows.bm;
     if (pf_n_groups * T > 0x7fffffffLL / 8) return fail(SSL_ERR_INVALID, "grid too large");
-    rows.items = (int)(pf_n_groups * T);
+    // K parts when the row grid is small (prefill_row_split) and the counters
+    // and workspace hold their arrivals and partial tiles (a call with less
+    // runs whole groups)
+    pm.ksplit = prefill_row_split(
+        pf_n_groups * T,
+        prefill_group_steps(nnz, n_chunks, K, block_p, pf_group, ssl_prefill_step_cols(dtype)), 0,
+        device_cus(), rows.bm, dtype);
+    const int64_t part_bytes = pm.ksplit * pf_n_groups * T * rows.bm * 64 * 4;
+    if (n_counters < ssl_bsr_addmm_counter_count(M, NB) || pf_n_groups > NB ||
+        part_bytes > workspace_bytes - need || part_bytes > 0x7fffffffLL)
+      pm.ksplit = 1;
+    if (pm.ksplit > 1) {
+      pm.kpart = (float*)((char*)workspace + need);
+      pm.karrive = counters + op_counters_min(M, NB);
+    }
+    rows.items = (int)(pf_n_groups * T * pm.ksplit);
     rows.off[1] = rows.items;
     return check_hip(prefill_launch_op(dtype, block_p, pf_group, rows, (hipStream_t)stream),
                      "bsr_addmm prefill launch");
@@ -716,15 +745,39 @@ int ssl_slr_forward_group(const void* x, int64_t ldx, int64_t M, int64_t m, int6
     rows.bm = prefill_row_tile(M, total_rows, G, block_p, cus, dtype, lat_wgs);
     // K parts: when the row grid is small (prefill_row_split) and every
     // member's workspace holds the partial tiles
-    int64_t items0 = 0, sp_steps = 0, n_grp = 0;
-    for (int i = 0; i < n_members; ++i)
-      if (members[i].NB > 0 && members[i].pf_n_groups > 0) {
-        items0 += members[i].pf_n_groups * ((M + rows.bm - 1) / rows.bm);
-        n_grp += members[i].pf_n_groups;
-        sp_steps += members[i].nnz * block_p / ssl_prefill_step_cols(dtype);
+    const int step_cols = ssl_prefill_step_cols(dtype);
+    int64_t n_grp = 0, grp_steps = 0;
+    int64_t lat_split = 0;  // the latent's workgroups when the rows split
+    for (int i = 0; i < n_members; ++i) {
+      const ssl_slr_member& mb = members[i];
+      if (mb.NB == 0) continue;
+      n_grp += mb.pf_n_groups;
+      grp_steps += mb.pf_n_groups *
+                   prefill_group_steps(mb.nnz, mb.n_chunks, m_pad, block_p, G, step_cols);
+      if (mb.r_pad > 0)
+        lat_split += TL * (mb.r_pad / 64) * prefill_latent_split(M, m_pad, mb.r_pad, dtype).split;
+    }
+    if (n_grp > 0) grp_steps /= n_grp;
+    int ksplit = prefill_row_split(n_grp * ((M + rows.bm - 1) / rows.bm), grp_steps, lat_split, cus,
+                                   rows.bm, dtype);
+    const int64_t short_items = n_grp * ((M + 63) / 64);
+    if (rows.bm == 64 && short_items >= cus && dtype != SSL_F32 && knobs.prefill_split == 0 &&
+        knobs.prefill_group == 0) {
+      // from one short workgroup a compute unit on, more narrow parts are better,
+      // and as many with 64×64 blocks, whose steps always load a whole weight
+      // tile: 4096×11008 with 64×64 at 50% (86 steps) at 256 rows narrow in two
+      // 48.7 µs, short in two 52.0 (Zipf 2048×8192 with 16×16 at 30% at 512: 58.7 /
+      // 53.3); 3200×8640 with 32×32 (101) at 384
+      // narrow in 3 58.0, short in two 62.1; 2:4 2048×8192 (128) at 600 narrow in
+      // 3 60.9, short whole 91.1. With fewer: 1600×8192 with 32×32 at 90% (127) at
+      // 512 rows (200 short) narrow in 3 61.4, short in two 55.5.
+      const int kn = prefill_row_split(n_grp * ((M + 127) / 128), grp_steps, lat_split, cus, 128,
+                                       dtype);
+      if (kn > ksplit || (kn == ksplit && kn > 1 && block_p == 64)) {
+        rows.bm = 128;
+        ksplit = kn;
       }
-    int ksplit = prefill_row_split(items0, n_grp > 0 ? sp_steps / n_grp : 0,
-                                   m_pad / ssl_prefill_step_cols(dtype), cus, rows.bm);
+    }
     for (int i = 0; i < n_members && ksplit > 1; ++i) {
       const ssl_slr_member& mb = members[i];
       if (mb.NB == 0) continue;

@@ -89,15 +89,20 @@ constexpr int kPartInts = 8;
 constexpr int kPrefillLatentRows = 64;
 constexpr int kPfLatArriveWord = 64;  // rank tiles ≤ 64 (r_pad ≤ 4096) for a latent split
 
-// K parts of a fused prefill call with few row workgroups: a grid of `items`
-// row workgroups under twice the CUs splits each row group's sparse steps in
-// up to 4 parts (at least 40 steps a part, `steps` the mean per group, the
-// parts at most twice the CUs; past half the CUs' worth of groups only parts
-// of 64 steps or more, or when the latent's steps are 1.5 times the group's),
-// and then the latent's in_features too (prefill_latent_split), so neither
-// leaves the other's critical path. 1 = no split.
-// lat_steps: the latent's steps over in_features.
-int prefill_row_split(int64_t items, int64_t steps, int64_t lat_steps, int n_cus, int bm);
+// Sparse steps of a group of block-rows: the union of `group` rows' blocks,
+// were nnz blocks spread evenly over rows × m_pad/block_p.
+int64_t prefill_group_steps(int64_t nnz, int64_t rows, int64_t m_pad, int block_p, int group,
+                            int step_cols);
+// K parts of a prefill call with few row workgroups: each row group's sparse
+// steps (`steps` a group) in up to 4 parts of at least 20 steps (28 for
+// 16-bit calls from one workgroup per compute unit on, 33 for the narrow tile),
+// as long as the parts are resident at once: with the latent's workgroups (`lat_items`, its K
+// chunks included) three a compute unit for the short tile, by themselves two
+// for the narrow one. The latent's in_features then split too
+// (prefill_latent_split), so neither leaves the other's critical path. 1 = no
+// split.
+int prefill_row_split(int64_t items, int64_t steps, int64_t lat_items, int n_cus, int bm,
+                      int dtype);
 struct PfLatentSplit {
   int split, chunk;
 };

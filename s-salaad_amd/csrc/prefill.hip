@@ -1075,34 +1075,59 @@ hipError_t launch_fused(const PfArgs& rows, const PfArgs& lat, int P, int G, hip
 
 }  // namespace
 
-// Parts of fewer steps lose more to the exchange of partial tiles (a store,
-// its acknowledgement, a count, a load: some µs) than they gain: 7B FFN
-// 11008×4096 (32 steps a group) at 256 rows 41.1 µs whole, 53.7 in two parts;
-// 4096×11008 (86 steps) 65.9 whole, 53.3 in two parts, 58.2 in three.
-constexpr int64_t kRowSplitMinSteps = 40;
-// Past half the CUs' worth of row groups, parts stack on compute units that
-// already run one: two parts pay only when each is long or the latent is what
-// they would otherwise wait for. Measured (whole -> auto parts, µs): 4096×11008
-// with 64×64 blocks (86 steps a group, 172-step latent) at 384 / 512 rows 66.1
-// -> 67.2 / 79.6 -> 66.7, at 640 (640 parts) 85.1 -> 96.9; with 16×16 (344
-// steps) at 512 134.5 -> 95.8; 2048×5461 with 32×32 (86 steps, 86-step latent)
-// at 512 / 640 / 768 rows 62.7 -> 56.1 / 65.2 -> 68.0 / 65.0 -> 70.6.
-constexpr int64_t kRowSplitLongSteps = 64;
+// A part shorter than this loses more to the exchange of partial tiles (a
+// store, its acknowledgement, a count, a load) than it gains: 64×64 tiles,
+// bf16, µs whole / 2 / 3 / 4 parts: 2048×2048 with 32×32 blocks at 50% (24
+// steps a group) at 256 rows 17.7 / 19.8 / 21.1 / 25.9; 1024×4096 (48) 25.2 /
+// 18.5 / 18.7 / 21.1; 2048×5461 (64) 49.6 / 38.3 / 33.9 / 38.4.
+constexpr int64_t kRowSplitMinSteps = 20;
+// Short 16-bit tiles from one workgroup per compute unit on share a unit's load
+// path and their parts have to be longer: 4096×11008 with 64×64 blocks at 30%
+// (52 steps) at 256 rows (256 workgroups) 39.9 whole, 42.9 in two parts;
+// 2048×5461 with 32×32 (64) at 512 rows 58.5 / 47.6. fp32 steps are bound by
+// their MFMAs, which parts spread: 1024×2048 with 32×32 (48) at 1024 rows (256
+// workgroups) 80.6 / 56.6.
+constexpr int64_t kRowSplitLongSteps = 28;
+// Narrow parts move more per step: 2048×5461 with 32×32 (64) at 768 rows 61.5
+// whole, 66.2 in two parts; the op's 4096×11008 with 64×64 (86) at 512 rows 60.4 /
+// 54.6; 3200×8640 with 32×32 (101) at 384 rows 68.3 / 63.6, in 3 parts 58.0.
+constexpr int64_t kRowSplitNarrowSteps = 33;
 
-int prefill_row_split(int64_t items, int64_t steps, int64_t lat_steps, int n_cus, int bm) {
+int64_t prefill_group_steps(int64_t nnz, int64_t rows, int64_t m_pad, int block_p, int group,
+                            int step_cols) {
+  const int64_t cols = m_pad / block_p;
+  if (rows <= 0 || cols <= 0) return 0;
+  const double absent = 1.0 - (double)nnz / ((double)rows * (double)cols);
+  double none = 1.0;
+  for (int g = 0; g < group; ++g) none *= absent > 0.0 ? absent : 0.0;
+  return (int64_t)((1.0 - none) * (double)(cols * block_p / step_cols) + 0.5);
+}
+
+int prefill_row_split(int64_t items, int64_t steps, int64_t lat_items, int n_cus, int bm,
+                      int dtype) {
   if (bm >= 256) return 1;  // the tall tile keeps its registers for its own steps
   const int64_t forced = debug_knobs().prefill_split;  // test hook
   if (forced == 1) return 1;
   if (forced >= 2) return (int)forced;
-  const int64_t slots = 2 * (int64_t)n_cus;
-  if (items <= 0 || items >= slots) return 1;
-  int64_t k = (slots + items - 1) / items;
-  if (k > 4) k = 4;
-  if (k > steps / kRowSplitMinSteps) k = steps / kRowSplitMinSteps;
-  while (k >= 2 && k * items > slots) --k;
-  if (k < 2) return 1;
-  if (2 * items > n_cus && steps / k < kRowSplitLongSteps && 2 * lat_steps < 3 * steps) return 1;
-  return (int)k;
+  if (items <= 0) return 1;
+  const bool narrow = bm > 64;
+  int64_t k = steps / (narrow ? kRowSplitNarrowSteps
+                       : dtype != SSL_F32 && items >= n_cus ? kRowSplitLongSteps
+                                                            : kRowSplitMinSteps);
+  // (three parts of 256 groups: the op's 4096×11008 at 256 rows 41.2 µs in two,
+  // 45.0; four of 128: 2048×8192 with 16×16 at 30% at 200 rows 32.5 in three, 33.5)
+  const int64_t most = narrow ? 4 : items >= n_cus ? 2 : 2 * items >= n_cus ? 3 : 4;
+  if (k > most) k = most;
+  // Every part resident at once, or the last ones run a round late. Short tiles
+  // take three workgroups a compute unit, the latent's included: 2048×5461 at
+  // 384 rows (192 groups, 144 latent chunks) in 3 parts 41.2 µs, in 4 50.3;
+  // 3200×8640 at 512 rows (400 groups) whole 73.3, in two 84.0. Narrow parts
+  // stop at two a unit: the op's 4096×11008 with 64×64 blocks at 512 rows (256
+  // groups) 60.4 / 54.6 in two parts, at 700 (384) 69.5 / 81.5.
+  while (k >= 2 && (narrow ? k * items > 2 * (int64_t)n_cus
+                           : k * items + lat_items > 3 * (int64_t)n_cus))
+    --k;
+  return k < 2 ? 1 : (int)k;
 }
 
 // The latent's K chunks when the rows split: chunks of at least 16 steps, at
@@ -1196,9 +1221,12 @@ int prefill_row_tile(int64_t M, int64_t n_rows, int group, int block_p, int n_cu
   // workgroups per compute unit (LLaMA-60M gate at 2048 rows: 58 -> 50 µs).
   if (dtype == SSL_F32 && narrow < 2 * n_cus) return 64;
   // A small grid: the short tile (64 × 64), twice the workgroups of the narrow
-  // one (2048×2048 with 32×32 blocks at 256 rows: 26.0 -> 22.7 µs; 4096×4096
-  // with 64×64 at 128 rows: 34.4 -> 31.7 µs).
-  if (narrow < n_cus / 2) return 64;
+  // one, up to one and a half a compute unit. Narrow / short, µs: 2048×2048 with
+  // 32×32 blocks at 256 rows (128 short workgroups) 22.0 / 17.7, 4096×4096 with
+  // 64×64 at 256 (256) 29.0 / 27.7, 4096×11008 at 30% density at 256 (256) 42.0 /
+  // 39.9 and at 384 (384) 46.7 / 45.9; at 512 rows (512) 49.3 / 54.4.
+  const int64_t small = ((M + 63) / 64) * groups;
+  if (2 * small <= 3 * (int64_t)n_cus) return 64;
   if (M <= 128) return 128;  // one token tile either way; the tall one's lower half past M
   // Rounds of the grid at the tile's workgroups per compute unit, the tall tile
   // (80 KiB of LDS: 2) against the narrow one (48 KiB: 3); a round of tall

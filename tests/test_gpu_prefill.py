@@ -236,6 +236,55 @@ def test_split_grouped_launch(k, tile, split, gpu_device):
     assert _counters_at_rest(gpu_device)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32],
+                         ids=["bf16", "f16", "f32"])
+@pytest.mark.parametrize("p,mode,k", [(16, SHORT, 2), (32, SHORT, 3), (32, NARROW, 4),
+                                      (64, SHORT, 4), (64, NARROW, 2)])
+def test_op_in_k_parts(dtype, p, mode, k, tile, split, gpu_device):
+    """The op's row groups in k parts: the parts' fp32 tiles summed in part order
+    by the last to arrive, which adds the old out. Skewed rows (groups with fewer
+    steps than parts), ragged token counts; the same bits on a repeated call, and
+    the counters back at zero."""
+    if dtype == torch.float32 and p == 64:
+        pytest.skip("fp32 prefill blocks are 16 or 32")
+    tile(mode)
+    split(k)
+    prob = make_problem(9 * p + 64, 40 * p, 64, p, 0.5, dtype, seed=p + k, skew=True)
+    crow, col, vt, act = orc.module_buffers(prob["crow"], prob["col"], prob["vals"])
+    act = act[1:]  # one row left out
+    dev = gpu_device
+    args = [torch.from_numpy(crow).to(dev), torch.from_numpy(col).to(dev), to_dev(vt, dtype, dev),
+            torch.from_numpy(act).to(dev)]
+    for M in (128, 333):
+        x = make_x(prob, M, seed=M)
+        out0 = np.random.default_rng(M).standard_normal((M, prob["NB"] * p))
+        out0 = torch.from_numpy(out0).to(dtype).double().numpy()
+        want = orc.bsr_addmm_inplace(out0, x, crow, col, vt, act)
+        outs = [to_dev(out0, dtype, dev) for _ in range(2)]
+        for out in outs:
+            torch.ops.ssalaad.tilelang_bsr_addmm_inplace_dense_(out, to_dev(x, dtype, dev), *args)
+        assert _counters_at_rest(dev), M
+        assert err(outs[0], want) <= TOL[dtype], M
+        assert torch.equal(outs[0], outs[1]), M
+
+
+@pytest.mark.parametrize("n,m,p,dtype,M", [
+    (1024, 4096, 32, torch.bfloat16, 200),   # 64 short workgroups, in parts
+    (4096, 11008, 64, torch.bfloat16, 256),  # 256 of them: narrow, in parts
+    (1024, 2048, 32, torch.float32, 1024),   # fp32, in two parts
+    (4096, 4096, 64, torch.bfloat16, 384),   # 384 of them: short, whole
+], ids=["short-parts", "narrow-parts", "f32-parts", "short-whole"])
+def test_tile_and_parts_of_small_grids(n, m, p, dtype, M, gpu_device):
+    """The library's own choice of tile and parts on either side of its rules."""
+    prob = make_problem(n, m, 128, p, 0.5, dtype, seed=n + M)
+    mod = make_module(prob, gpu_device)
+    x = make_x(prob, M, seed=M)
+    y = mod(to_dev(x, dtype, gpu_device))
+    torch.cuda.synchronize()
+    assert err(y, oracle_y(prob, x)) <= TOL[dtype]
+    assert _counters_at_rest(gpu_device)
+
+
 # -------------------------------------------- full size, library's choice --
 
 
