@@ -679,6 +679,30 @@ def test_encoder_structure_is_bit_exact(dtype, pq, gpu_device):
     assert np.array_equal(k_vt.cpu().view(bits).numpy(), want_bits.transpose(0, 2, 1))
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("p,q,nbk", [(16, 16, 1100), (64, 64, 9), (32, 512, 5), (128, 16, 33),
+                                     (48, 32, 70), (32, 48, 1030), (96, 80, 6)])
+def test_encoder_fill_places_every_block(dtype, p, q, nbk, gpu_device):
+    """Kept columns and both value copies for power-of-two and other blocks,
+    whole small blocks and several slabs a block, rows of more than one 1024-column
+    segment, an empty row and a full one: bit for bit against torch."""
+    g = torch.Generator().manual_seed(p + q + nbk)
+    nb = 3
+    keep = torch.rand(nb, nbk, generator=g) < 0.5
+    keep[0], keep[1] = False, True
+    S = torch.randn(nb, p, nbk, q, generator=g) * keep[:, None, :, None]
+    S = S.reshape(nb * p, nbk * q).to(dtype)
+    rows, cols = keep.nonzero(as_tuple=True)
+    blocks = S.view(nb, p, nbk, q)[rows, :, cols]  # (nnz, p, q)
+    crow, col, vt, act = ssalaad_amd.encode_for_kernels(S.to(gpu_device), p, q)
+    assert crow.cpu().tolist() == [0] + keep.sum(1).cumsum(0).tolist()
+    assert torch.equal(col.cpu().long(), cols)
+    assert torch.equal(vt.cpu(), blocks.transpose(1, 2))
+    assert act.cpu().tolist() == [1, 2]
+    b = ssalaad_amd.dense_to_bsr(S.to(gpu_device), p, q)
+    assert torch.equal(b.values().cpu(), blocks)
+
+
 def test_encoder_feeds_the_module(gpu_device):
     """Dense S handed to the factory goes through the device encoder."""
     prob = make_problem(128, 192, 16, 32, 0.4, torch.bfloat16, seed=2)
