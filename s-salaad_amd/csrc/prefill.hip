@@ -1115,8 +1115,10 @@ int prefill_row_split(int64_t items, int64_t steps, int64_t lat_items, int n_cus
                        : dtype != SSL_F32 && items >= n_cus ? kRowSplitLongSteps
                                                             : kRowSplitMinSteps);
   // (three parts of 256 groups: the op's 4096×11008 at 256 rows 41.2 µs in two,
-  // 45.0; four of 128: 2048×8192 with 16×16 at 30% at 200 rows 32.5 in three, 33.5)
-  const int64_t most = narrow ? 4 : items >= n_cus ? 2 : 2 * items >= n_cus ? 3 : 4;
+  // 45.0; four of 128 groups: 2048×8192 at 200 rows with 16×16 at 30% (97 steps)
+  // 32.5 in three, 33.5, and 2:4 (128) 40.4 in three, 37.9)
+  const bool few = 2 * items >= n_cus && steps < 4 * kRowSplitLongSteps;
+  const int64_t most = narrow ? 4 : items >= n_cus ? 2 : few ? 3 : 4;
   if (k > most) k = most;
   // Every part resident at once, or the last ones run a round late. Short tiles
   // take three workgroups a compute unit, the latent's included: 2048×5461 at
