@@ -293,6 +293,23 @@ def check(rc: int, what: str) -> None:
     raise RuntimeError(msg)
 
 
+# What a launcher (hostcall) returns when nothing reached the stream: a raised
+# status word (−1) and the entry points' own checks, all made before any launch.
+_NOT_ISSUED = (-1, SSL_ERR_INVALID, SSL_ERR_UNSUPPORTED, SSL_ERR_WORKSPACE, SSL_ERR_CAPACITY)
+
+
+def issued(rc: int, what: str) -> bool:
+    """Whether a launcher's call was issued; False when it was refused before
+    any launch, so that another path may take it. A HIP error raises: it is read
+    after the launch and may stem from an earlier call of the thread, so the
+    kernel may be on the stream already."""
+    if rc == SSL_OK:
+        return True
+    if rc not in _NOT_ISSUED:
+        check(rc, what)
+    return False
+
+
 def ptr(t: torch.Tensor | None) -> int | None:
     return None if t is None else t.data_ptr()
 

@@ -92,10 +92,15 @@ def _validated_host_structure(crow, col, active_rows, nnz_values, NB_K):
     return crow_h.astype(np.int32), act_h.astype(np.int32)
 
 
+def _versions(crow, col, active_rows) -> tuple:
+    """What a structure's plans and launchers were built from."""
+    return (crow._version, col._version, active_rows._version, col.data_ptr(),
+            active_rows.data_ptr())
+
+
 def _plan_for(crow, col, active_rows, values, NB_K, block_p, block_q, M, elem_bytes,
               prefill=None):
-    versions = (crow._version, col._version, active_rows._version, col.data_ptr(),
-                active_rows.data_ptr(), values.shape[0], NB_K)
+    versions = _versions(crow, col, active_rows) + (values.shape[0], NB_K)
     sp = getattr(crow, _PLAN_ATTR, None)
     if (
         sp is None
@@ -203,11 +208,11 @@ def _repeat(out, x, crow, col, values, active) -> bool:
     if (out.dtype is not values.dtype or x.dtype is not values.dtype or out.device != dev
             or x.device != dev or values.device != dev
             or not (out.is_contiguous() and x.is_contiguous() and values.is_contiguous())
-            or sp.versions[:5] != (crow._version, col._version, active._version, col.data_ptr(),
-                                   active.data_ptr())):
+            or sp.versions[:-2] != _versions(crow, col, active)):
         return False
     o, xp, v = out.data_ptr(), x.data_ptr(), values.data_ptr()
-    return (o | xp | v) % 16 == 0 and hit[1].launch(o, xp, v) == 0
+    return (o | xp | v) % 16 == 0 and _lib.issued(hit[1].launch(o, xp, v),
+                                                  "ssl_bsr_addmm_inplace")
 
 
 def bsr_addmm_inplace_(

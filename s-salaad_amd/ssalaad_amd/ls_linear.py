@@ -383,11 +383,11 @@ def _relaunch(states, x: torch.Tensor, out_features):
     if len(pads) == 1:
         n, pad = out_features[0], pads[0]
         y = torch.empty((*lead, pad), dtype=x.dtype, device=x.device)
-        if launcher.launch(xp, y.data_ptr()) != 0:
+        if not _lib.issued(launcher.launch(xp, y.data_ptr()), "ssl_slr_forward_group"):
             return None
         return (y if n == pad else y[..., :n],)
     ys = [torch.empty((*lead, pad), dtype=x.dtype, device=x.device) for pad in pads]
-    if launcher.launch(xp, *[y.data_ptr() for y in ys]) != 0:
+    if not _lib.issued(launcher.launch(xp, *[y.data_ptr() for y in ys]), "ssl_slr_forward_group"):
         return None
     return [y if n == pad else y[..., :n] for y, n, pad in zip(ys, out_features, pads)]
 

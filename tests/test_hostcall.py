@@ -1,0 +1,100 @@
+"""The kept launchers of eager calls (hostcall), without a GPU: stub launchers
+stand in for the compiled ones, CPU tensors for the device's."""
+
+import pytest
+import torch
+
+from ssalaad_amd import LRSLinearGroup, _lib, _runtime, addmm_inplace, ls_linear
+
+
+class Stub:
+    """A launcher that counts its calls and returns a given status."""
+
+    def __init__(self, rc=0):
+        self.rc, self.calls = rc, 0
+
+    def launch(self, *args):
+        self.calls += 1
+        return self.rc
+
+
+@pytest.fixture(autouse=True)
+def no_device(monkeypatch):
+    """The device queries of the call path, answered as for CPU tensors."""
+    monkeypatch.setattr(torch._C, "_cuda_getDevice", lambda: None)
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda i: 0)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+
+
+def kept_op_call(stub, nb=2, p=16):
+    """Arguments of an op call whose launcher is kept."""
+    crow = torch.arange(nb + 1, dtype=torch.int32)
+    col = torch.zeros(nb, dtype=torch.int32)
+    act = torch.arange(nb, dtype=torch.int32)
+    vals = torch.zeros(nb, p, p)
+    out, x = torch.zeros(3, nb * p), torch.zeros(3, p)
+    sp = addmm_inplace._StructPlan(addmm_inplace._versions(crow, col, act) + (nb, 1), col, act, 1)
+    sp.calls[(out.shape, x.shape, vals.shape, vals.dtype, 0)] = (_runtime.generation(), stub)
+    setattr(crow, addmm_inplace._PLAN_ATTR, sp)
+    return out, x, crow, col, vals, act
+
+
+def kept_linear(stub, n=64, m=64, tokens=3):
+    """A low-rank linear whose launcher for `tokens` rows is kept."""
+    mod = ls_linear._LRSLinearLR(torch.randn(n, 16), torch.randn(16, m), in_features=m,
+                                 out_features=n)
+    st = mod._state = ls_linear._KernelState(mod, torch.device("cpu"))
+    st._launchers[(tokens, 0, id(st))] = (_runtime.generation(), None, stub, (st,), (n,))
+    return mod, torch.randn(tokens, m)
+
+
+def kept_group(stub, n=64, m=64, tokens=3):
+    mods = [kept_linear(None, n, m)[0] for _ in range(2)]
+    sts = [mod._state for mod in mods]
+    sts[0]._launchers[(tokens, 0, *map(id, sts))] = (_runtime.generation(), None, stub, tuple(sts),
+                                                     (n, n))
+    return LRSLinearGroup(*mods), torch.randn(tokens, m)
+
+
+# Argument errors are found before any launch; a HIP error is read after it.
+REFUSED = [-1, _lib.SSL_ERR_INVALID, _lib.SSL_ERR_UNSUPPORTED, _lib.SSL_ERR_WORKSPACE]
+
+
+def test_op_call_with_a_hip_error_is_not_issued_again():
+    """The kernel may be on the stream already (a stale error of the thread is
+    reported too), and a second one would add x·Sᵀ twice."""
+    stub = Stub(_lib.SSL_ERR_HIP)
+    with pytest.raises(RuntimeError, match="ssl_bsr_addmm_inplace"):
+        addmm_inplace._repeat(*kept_op_call(stub))
+    assert stub.calls == 1
+
+
+@pytest.mark.parametrize("rc", REFUSED)
+def test_refused_op_call_takes_the_full_path(rc):
+    stub = Stub(rc)
+    assert addmm_inplace._repeat(*kept_op_call(stub)) is False
+    assert stub.calls == 1
+    stub = Stub(0)
+    assert addmm_inplace._repeat(*kept_op_call(stub)) is True
+
+
+@pytest.mark.parametrize("make", [kept_linear, kept_group])
+def test_module_call_with_a_hip_error_raises(make, monkeypatch):
+    stub = Stub(_lib.SSL_ERR_HIP)
+    mod, x = make(stub)
+    monkeypatch.setattr(ls_linear, "_launch", lambda *a: pytest.fail("issued again"))
+    with pytest.raises(RuntimeError, match="ssl_slr_forward_group"):
+        mod(x)
+    assert stub.calls == 1
+
+
+@pytest.mark.parametrize("make", [kept_linear, kept_group])
+@pytest.mark.parametrize("rc", [0] + REFUSED)
+def test_module_call_uses_the_kept_launcher_or_the_full_path(make, rc, monkeypatch):
+    stub = Stub(rc)
+    mod, x = make(stub)
+    full = []
+    monkeypatch.setattr(ls_linear, "_launch", lambda *a: full.append(1) or [x])
+    monkeypatch.setattr(ls_linear._KernelState, "forward", lambda *a: full.append(1) or x)
+    mod(x)
+    assert stub.calls == 1 and len(full) == (0 if rc == 0 else 1)
