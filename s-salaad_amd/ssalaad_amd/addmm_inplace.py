@@ -298,9 +298,19 @@ def bsr_addmm_inplace_(
     dt = _lib.dtype_code(out_inplace.dtype)
     dev = out_inplace.device
     with torch.cuda.device(dev):
+        generation = _runtime.generation()
         ws = _runtime.workspace(dev, lib.ssl_bsr_addmm_workspace_size(M, NB, block_p, plan.n_slots))
         cnt = _runtime.counters(dev, lib.ssl_bsr_addmm_counter_count(M, NB))
         vals_pq = _values_pq(values, vals) if pf else None
+        # built before the launch: nothing after it may raise for want of it
+        launcher = None
+        if (pf is None and target is out_inplace and out_inplace.is_contiguous()
+                and x.is_contiguous() and col is col_indices and dev.index is not None):
+            launcher = _lib.hostcall().OpCall(
+                _lib.entry_address("ssl_bsr_addmm_inplace"), _runtime.status_word(dev).host_ptr,
+                N, K, col.data_ptr(), vals.shape[0], plan.table.data_ptr(), plan.n_chunks,
+                plan.n_slots, M, N, K, NB, block_p, block_q, dt, cnt.data_ptr(), cnt.numel(),
+                ws.data_ptr(), ws.numel(), _lib.stream_ptr(dev))
         rc = lib.ssl_bsr_addmm_inplace(
             target.data_ptr(), target.stride(0), x.data_ptr(), x.stride(0), col.data_ptr(),
             vals.data_ptr(), vals.shape[0], plan.table.data_ptr(), plan.n_chunks, plan.n_slots,
@@ -311,18 +321,12 @@ def bsr_addmm_inplace_(
             _lib.stream_ptr(dev),
         )
     _lib.check(rc, "ssl_bsr_addmm_inplace")
-    if (pf is None and target is out_inplace and out_inplace.is_contiguous()
-            and x.is_contiguous() and col is col_indices and dev.index is not None):
-        sp = getattr(crow_indices, _PLAN_ATTR)
-        if len(sp.calls) >= _MAX_CALLS:
-            sp.calls.clear()
-        sp.calls[(out_inplace.shape, x.shape, values.shape, values.dtype, _lib.stream_ptr(dev))] = (
-            _runtime.generation(),
-            _lib.hostcall().OpCall(
-                _lib.entry_address("ssl_bsr_addmm_inplace"), _runtime.status_word(dev).host_ptr,
-                N, K, col.data_ptr(), vals.shape[0], plan.table.data_ptr(), plan.n_chunks,
-                plan.n_slots, M, N, K, NB, block_p, block_q, dt, cnt.data_ptr(), cnt.numel(),
-                ws.data_ptr(), ws.numel(), _lib.stream_ptr(dev)))
+    if launcher is not None:
+        calls = getattr(crow_indices, _PLAN_ATTR).calls
+        if len(calls) >= _MAX_CALLS:
+            calls.clear()
+        calls[(out_inplace.shape, x.shape, values.shape, values.dtype, _lib.stream_ptr(dev))] = (
+            generation, launcher)
     if target is not out_inplace:
         out_inplace.copy_(target)
 

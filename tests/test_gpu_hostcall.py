@@ -142,6 +142,25 @@ def test_repeated_op_calls(tokens, gpu_device):
     assert torch.equal(out[:, -32:], out0[:, -32:]) and torch.equal(out[:, :-32], first[:, :-32])
 
 
+def test_op_without_the_host_call_path_leaves_out_as_it_was(gpu_device, monkeypatch):
+    """A missing extension is found before the launch: out keeps its bits, so a
+    call made again after the error adds x·Sᵀ once."""
+    mod, _ = _linear(5, bias=False)
+    args = [t.clone() for t in (mod.S_crow, mod.S_col, mod.S_values, mod.S_active_rows)]
+    x = torch.randn(3, 160, device="cuda").to(torch.bfloat16)
+    out = torch.randn(3, 192, device="cuda").to(torch.bfloat16)
+    before = out.clone()
+
+    def missing():
+        raise RuntimeError("the host call path is not built")
+
+    monkeypatch.setattr(_lib, "hostcall", missing)
+    with pytest.raises(RuntimeError, match="not built"):
+        torch.ops.ssalaad.tilelang_bsr_addmm_inplace_dense_(out, x, *args)
+    torch.cuda.synchronize()
+    assert torch.equal(out, before)
+
+
 def test_launchers_check_their_arguments():
     h = _lib.hostcall()
     with pytest.raises(ValueError):
