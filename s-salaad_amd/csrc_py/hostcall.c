@@ -216,7 +216,7 @@ typedef int (*op_fn)(void*, int64_t, const void*, int64_t, const int32_t*, const
 typedef struct {
   PyObject_HEAD
   op_fn fn;
-  const volatile uint64_t* status;
+  const volatile uint64_t* status; /* NULL: the device has no status word (yet) */
   int64_t ldo, ldx, nnz, n_chunks, n_slots, M, N, K, NB, n_counters, ws_bytes;
   int32_t p, q, dtype;
   const int32_t *col, *plan;
@@ -234,7 +234,7 @@ static PyObject* op_new(PyTypeObject* type, PyObject* args, PyObject* kw) {
     if (!PyErr_Occurred()) PyErr_SetString(PyExc_TypeError, "OpCall takes no keywords");
     return NULL;
   }
-  if (!fn || !status) {
+  if (!fn) {
     PyErr_SetString(PyExc_ValueError, "OpCall: bad arguments");
     return NULL;
   }
@@ -263,7 +263,7 @@ static PyObject* op_launch(OpCall* o, PyObject* const* args, Py_ssize_t nargs) {
   const void* x = (const void*)(uintptr_t)PyLong_AsUnsignedLongLong(args[1]);
   const void* values = (const void*)(uintptr_t)PyLong_AsUnsignedLongLong(args[2]);
   if (PyErr_Occurred()) return NULL;
-  if (*o->status != 0) return PyLong_FromLong(-1);
+  if (o->status && *o->status != 0) return PyLong_FromLong(-1);
   int rc;
   Py_BEGIN_ALLOW_THREADS
   rc = o->fn(out, o->ldo, x, o->ldx, o->col, values, o->nnz, o->plan, o->n_chunks, o->n_slots, NULL,

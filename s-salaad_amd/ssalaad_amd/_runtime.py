@@ -280,8 +280,9 @@ class DevicePlan:
         return int(self._exchange[:8].view(torch.int64)[0].item())
 
 
-# Counts every replacement of a pool buffer or exchange area: a call bound to
-# them at one value is bound to the live ones while the value stands.
+# Counts every replacement of a pool buffer or exchange area and every new
+# status word: a call bound to them at one value is bound to the live ones while
+# the value stands.
 _generation = 0
 
 
@@ -367,7 +368,16 @@ def status_word(device: torch.device) -> StatusWord:
         with torch.cuda.device(idx):
             w = StatusWord()
         _STATUS[idx] = w
+        _replaced()  # launchers made without it check it from now on
     return w
+
+
+def status_address(device: torch.device) -> int:
+    """The host address of the device's status word, or 0 while it has none (no
+    fused call so far). Allocates nothing: the op's calls never wait, and a first
+    one under graph capture may not allocate pinned memory."""
+    w = _STATUS.get(_index(device))
+    return 0 if w is None else w.host_ptr
 
 
 def check_status(device: torch.device) -> None:

@@ -307,7 +307,7 @@ def bsr_addmm_inplace_(
         if (pf is None and target is out_inplace and out_inplace.is_contiguous()
                 and x.is_contiguous() and col is col_indices and dev.index is not None):
             launcher = _lib.hostcall().OpCall(
-                _lib.entry_address("ssl_bsr_addmm_inplace"), _runtime.status_word(dev).host_ptr,
+                _lib.entry_address("ssl_bsr_addmm_inplace"), _runtime.status_address(dev),
                 N, K, col.data_ptr(), vals.shape[0], plan.table.data_ptr(), plan.n_chunks,
                 plan.n_slots, M, N, K, NB, block_p, block_q, dt, cnt.data_ptr(), cnt.numel(),
                 ws.data_ptr(), ws.numel(), _lib.stream_ptr(dev))

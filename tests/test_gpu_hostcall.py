@@ -5,7 +5,7 @@ status — takes the full path again with the full path's results and errors."""
 import pytest
 import torch
 
-from ssalaad_amd import LRSLinear, LRSLinearGroup, _lib, _runtime, clear_wait_status
+from ssalaad_amd import LRSLinear, LRSLinearGroup, _lib, _runtime, clear_wait_status, prepare_bsr_addmm
 
 pytestmark = pytest.mark.gpu
 
@@ -159,6 +159,43 @@ def test_op_without_the_host_call_path_leaves_out_as_it_was(gpu_device, monkeypa
         torch.ops.ssalaad.tilelang_bsr_addmm_inplace_dense_(out, x, *args)
     torch.cuda.synchronize()
     assert torch.equal(out, before)
+
+
+def test_first_op_call_under_capture_allocates_no_pinned_memory(gpu_device, monkeypatch):
+    """On a device without a status word (no fused call so far) the op makes
+    none: pinned memory may not be allocated while a stream is capturing. Once
+    there is one, repeated calls check it."""
+    mod, _ = _linear(6, bias=False)
+    args = [t.clone() for t in (mod.S_crow, mod.S_col, mod.S_values, mod.S_active_rows)]
+    prepare_bsr_addmm(*args, 160)
+    op = torch.ops.ssalaad.tilelang_bsr_addmm_inplace_dense_
+    x = torch.randn(3, 160, device="cuda").to(torch.bfloat16)
+    out0 = torch.randn(3, 192, device="cuda").to(torch.bfloat16)
+    want = out0.clone()
+    op(want, x, *args)
+    args[0] = args[0].clone()  # no kept launchers
+    prepare_bsr_addmm(*args, 160)
+    monkeypatch.setattr(_runtime, "_STATUS", {})
+    real = _runtime.StatusWord
+    monkeypatch.setattr(_runtime, "StatusWord", lambda: pytest.fail("allocated"))
+    out = out0.clone()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        op(out, x, *args)
+    for _ in range(3):
+        out.copy_(out0)
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+    op(out.copy_(out0), x, *args)
+    monkeypatch.setattr(_runtime, "StatusWord", real)
+    word = _runtime.status_word(x.device)
+    word._word.value = 1
+    with pytest.raises(RuntimeError, match="gave up"):
+        op(out, x, *args)
+    word.clear()
+    op(out.copy_(out0), x, *args)
+    assert torch.equal(out, want)
 
 
 def test_launchers_check_their_arguments():

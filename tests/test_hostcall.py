@@ -1,6 +1,8 @@
 """The kept launchers of eager calls (hostcall), without a GPU: stub launchers
 stand in for the compiled ones, CPU tensors for the device's."""
 
+import contextlib
+
 import pytest
 import torch
 
@@ -98,3 +100,16 @@ def test_module_call_uses_the_kept_launcher_or_the_full_path(make, rc, monkeypat
     monkeypatch.setattr(ls_linear._KernelState, "forward", lambda *a: full.append(1) or x)
     mod(x)
     assert stub.calls == 1 and len(full) == (0 if rc == 0 else 1)
+
+
+def test_new_status_word_drops_the_launchers_made_without_it(monkeypatch):
+    monkeypatch.setattr(_runtime, "_STATUS", {})
+    monkeypatch.setattr(_runtime, "StatusWord", lambda: type("W", (), dict(host_ptr=64))())
+    monkeypatch.setattr(torch.cuda, "device", lambda i: contextlib.nullcontext())
+    dev = torch.device("cuda", 0)
+    assert _runtime.status_address(dev) == 0
+    stub = Stub()
+    args = kept_op_call(stub)
+    _runtime.status_word(dev)
+    assert _runtime.status_address(dev) == 64
+    assert addmm_inplace._repeat(*args) is False and stub.calls == 0
