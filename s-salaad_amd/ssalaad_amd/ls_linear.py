@@ -130,6 +130,13 @@ class _KernelState:
         self._pf_plans: dict[int, _runtime.DevicePrefillPlan] = {}
         self._values_pq: torch.Tensor | None = None
 
+    def views(self, mod: "_LRSLinearBase") -> bool:
+        """Whether mod.A still has this view's dtype and device: a reinterpreted
+        A keeps its pointer and version, and the calls it refuses are refused by
+        the full path."""
+        A = mod._buffers["A"]
+        return A.dtype is self.dtype and A.device == self.device
+
     def _padded(self, t: torch.Tensor, rows: int, cols: int) -> torch.Tensor:
         if t.shape == (rows, cols) and t.is_contiguous() and t.data_ptr() % 16 == 0:
             return t
@@ -523,8 +530,9 @@ class _LRSLinearBase(nn.Module):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         st = self._state
-        if (st is not None and x.dtype is st.dtype and x.shape[-1] == self.in_features
-                and x.device == st.device and st.watch.unchanged(self._buffers)):
+        if (st is not None and st.watch.unchanged(self._buffers) and st.views(self)
+                and x.dtype is st.dtype and x.shape[-1] == self.in_features
+                and x.device == st.device):
             out = _relaunch((st,), x, (self.out_features,))
             if out is not None:
                 return out[0]
@@ -743,7 +751,7 @@ class LRSLinearGroup(nn.Module):
         states, outf = [], []
         for mod in self.members._modules.values():
             st = mod._state
-            if st is None or not st.watch.unchanged(mod._buffers):
+            if st is None or not (st.watch.unchanged(mod._buffers) and st.views(mod)):
                 return None
             states.append(st)
             outf.append(mod.out_features)

@@ -113,3 +113,23 @@ def test_new_status_word_drops_the_launchers_made_without_it(monkeypatch):
     _runtime.status_word(dev)
     assert _runtime.status_address(dev) == 64
     assert addmm_inplace._repeat(*args) is False and stub.calls == 0
+
+
+@pytest.mark.parametrize("member", [0, 1])
+def test_reinterpreted_weights_are_refused_as_on_the_full_path(member, monkeypatch):
+    """A view of A in another dtype keeps A's pointer and version."""
+    stub = Stub()
+    grp, x = kept_group(stub)
+    monkeypatch.setattr(ls_linear, "_launch", lambda *a: pytest.fail("checks passed"))
+    mod = grp.members[member]
+    mod._kernel = lambda: pytest.fail("checks passed") if member == 0 else _lib.dtype_code(mod.A.dtype)
+    mod.A = mod.A.view(torch.int32)
+    with pytest.raises(TypeError):
+        grp(x)
+    assert stub.calls == 0
+
+    mod, x = kept_linear(stub)
+    mod.A = mod.A.view(torch.int32)
+    with pytest.raises(TypeError, match="input dtype"):
+        mod(x)
+    assert stub.calls == 0
