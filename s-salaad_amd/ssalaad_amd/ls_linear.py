@@ -512,6 +512,11 @@ class _LRSLinearBase(nn.Module):
         self._state = None  # weights moved or cast: rebuild the kernel view lazily
         return super()._apply(fn, recurse=recurse)
 
+    def __getstate__(self) -> dict:
+        # the kernel view holds raw pointers and compiled objects: a copy of the
+        # module (deepcopy, pickle) builds its own
+        return {**self.__dict__, "_state": None}
+
     def _weights_key(self) -> tuple:
         """Identity and in-place version of every buffer the kernel view is
         built from (the reference module reads its buffers on every forward;

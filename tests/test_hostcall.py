@@ -2,6 +2,8 @@
 stand in for the compiled ones, CPU tensors for the device's."""
 
 import contextlib
+import copy
+import pickle
 
 import pytest
 import torch
@@ -133,3 +135,13 @@ def test_reinterpreted_weights_are_refused_as_on_the_full_path(member, monkeypat
     with pytest.raises(TypeError, match="input dtype"):
         mod(x)
     assert stub.calls == 0
+
+
+def test_modules_with_a_kernel_view_can_be_copied():
+    """A copy has the same buffers and no kernel view of its own yet."""
+    mod, _ = kept_linear(Stub())
+    for twin in (copy.deepcopy(mod), pickle.loads(pickle.dumps(mod))):
+        assert twin._state is None and mod._state is not None
+        assert torch.equal(twin.A, mod.A) and twin.A.data_ptr() != mod.A.data_ptr()
+    grp, _ = kept_group(Stub())
+    assert [m._state for m in copy.deepcopy(grp).members] == [None, None]
