@@ -262,12 +262,13 @@ class DevicePlan:
         zeros, which is a valid state for the next call; the outgrown area is
         kept alive with the plan, since a graph captured earlier replays into it.
         """
-        if self._exchange is None or self._exchange.numel() < nbytes:
-            if self._exchange is not None:
-                self._retired.append(self._exchange)
-            _replaced()
+        old = self._exchange
+        if old is None or old.numel() < nbytes:
             self._exchange = torch.zeros(max(int(nbytes), 256), dtype=torch.uint8,
                                          device=self.table.device)
+            if old is not None:
+                self._retired.append(old)
+                _replaced()
         return self._exchange
 
     def wait_status(self) -> int:
@@ -282,7 +283,9 @@ class DevicePlan:
 
 # Counts every replacement of a pool buffer or exchange area and every new
 # status word: a call bound to them at one value is bound to the live ones while
-# the value stands.
+# the value stands. A first buffer replaces none (nothing is bound to it yet),
+# and the count follows the swap: whoever still read the old buffer read the old
+# count before it.
 _generation = 0
 
 
@@ -311,12 +314,14 @@ def _grown(pool, key, n, dtype, device, minimum):
     buf = pool.get(key)
     if buf is None or buf.numel() < n:
         size = max(int(n), minimum)
-        if buf is not None:
-            size = max(size, 2 * buf.numel())
-            _RETIRED.append(buf)
-        _replaced()
+        old = buf
+        if old is not None:
+            size = max(size, 2 * old.numel())
         buf = torch.zeros(size, dtype=dtype, device=device)
         pool[key] = buf
+        if old is not None:
+            _RETIRED.append(old)
+            _replaced()
     return buf
 
 

@@ -100,8 +100,10 @@ def test_groups_streams_and_grown_pools(gpu_device):
             assert all(torch.equal(u, v) for u, v in zip(grp(x), first))
     side.synchronize()
     before = _runtime.generation()
-    big = torch.randn(400, 160, device="cuda").to(torch.bfloat16)  # a larger exchange area
-    grp(big)
+    big = torch.randn(400, 160, device="cuda").to(torch.bfloat16)
+    for u, v in zip(grp(big[:3]), grp(big)):
+        assert u.shape[0] == 3 and v.shape[0] == 400
+    _runtime.workspace(x.device, _runtime.workspace(x.device, 1).numel() + 1)  # a grown pool
     assert _runtime.generation() > before
     for _ in range(2):
         assert all(torch.equal(u, v) for u, v in zip(grp(x), first))

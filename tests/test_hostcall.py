@@ -5,6 +5,7 @@ import contextlib
 import copy
 import pickle
 
+import numpy as np
 import pytest
 import torch
 
@@ -145,3 +146,26 @@ def test_modules_with_a_kernel_view_can_be_copied():
         assert torch.equal(twin.A, mod.A) and twin.A.data_ptr() != mod.A.data_ptr()
     grp, _ = kept_group(Stub())
     assert [m._state for m in copy.deepcopy(grp).members] == [None, None]
+
+
+def test_generation_counts_replaced_buffers_only(monkeypatch):
+    """A first buffer of another stream, plan or device drops no launcher; a
+    replaced one does, once the new one is in place."""
+    cpu = torch.device("cpu")
+    seen = []
+    monkeypatch.setattr(_runtime, "_RETIRED", [])
+    pool = {}
+    real = _runtime._replaced
+    monkeypatch.setattr(_runtime, "_replaced", lambda: (seen.append(pool[0].numel()), real()))
+    before = _runtime.generation()
+    small = _runtime._grown(pool, 0, 10, torch.int32, cpu, 16)
+    assert small.numel() == 16 and _runtime.generation() == before
+    assert _runtime._grown(pool, 0, 12, torch.int32, cpu, 16) is small
+    assert _runtime._grown(pool, 0, 17, torch.int32, cpu, 16).numel() == 32
+    assert seen == [32] and _runtime.generation() == before + 1 and _runtime._RETIRED == [small]
+
+    plan = _runtime.DevicePlan(np.zeros((1, 8), np.int32), 1, 0, cpu)
+    seen.clear()
+    area = plan.exchange(512)
+    assert not seen and plan.exchange(300) is area
+    assert plan.exchange(1024) is not area and len(seen) == 1 and plan._retired == [area]
