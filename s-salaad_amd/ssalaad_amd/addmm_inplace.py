@@ -94,7 +94,7 @@ def _validated_host_structure(crow, col, active_rows, nnz_values, NB_K):
 
 def _versions(crow, col, active_rows) -> tuple:
     """What a structure's plans and launchers were built from."""
-    return (crow._version, col._version, active_rows._version, col.data_ptr(),
+    return (crow._version, col._version, active_rows._version, crow.data_ptr(), col.data_ptr(),
             active_rows.data_ptr())
 
 

@@ -169,3 +169,18 @@ def test_generation_counts_replaced_buffers_only(monkeypatch):
     area = plan.exchange(512)
     assert not seen and plan.exchange(300) is area
     assert plan.exchange(1024) is not area and len(seen) == 1 and plan._retired == [area]
+
+
+@pytest.mark.parametrize("which", [2, 3, 5], ids=["crow", "col", "active"])
+def test_replaced_structure_takes_the_full_path(which):
+    """A structure tensor given other data keeps its identity and version; the
+    full path checks the new structure (a crow of other length is refused there)."""
+    stub = Stub()
+    args = kept_op_call(stub)
+    assert addmm_inplace._repeat(*args) is True
+    args[which].data = torch.cat([args[which], args[which][-1:]])
+    assert addmm_inplace._repeat(*args) is False and stub.calls == 1
+    stub = Stub()
+    args = kept_op_call(stub)
+    args[which].add_(0)
+    assert addmm_inplace._repeat(*args) is False and stub.calls == 0
