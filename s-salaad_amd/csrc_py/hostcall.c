@@ -69,23 +69,29 @@ static PyObject* watch_new(PyTypeObject* type, PyObject* args, PyObject* kw) {
   }
   Watch* w = (Watch*)type->tp_alloc(type, 0);
   if (!w) return NULL;
-  const Py_ssize_t n = PyDict_Size(d);
-  w->items = (Item*)PyMem_Calloc(n ? n : 1, sizeof(Item));
+  /* a list of its own: a tensor's methods may change the dict */
+  PyObject* pairs = PyDict_Items(d);
+  const Py_ssize_t n = pairs ? PyList_GET_SIZE(pairs) : 0;
+  w->items = pairs ? (Item*)PyMem_Calloc(n ? n : 1, sizeof(Item)) : NULL;
   if (!w->items) {
+    if (pairs) PyErr_NoMemory();
+    Py_XDECREF(pairs);
     Py_DECREF(w);
-    return PyErr_NoMemory();
+    return NULL;
   }
-  PyObject *key, *t;
-  Py_ssize_t pos = 0;
-  while (w->n < n && PyDict_Next(d, &pos, &key, &t)) {
+  while (w->n < n) {
+    PyObject* pair = PyList_GET_ITEM(pairs, w->n);
+    PyObject* t = PyTuple_GET_ITEM(pair, 1);
     Item* it = &w->items[w->n++];
-    it->name = Py_NewRef(key);
+    it->name = Py_NewRef(PyTuple_GET_ITEM(pair, 0));
     it->present = t != Py_None;
     if (it->present && tensor_state(t, &it->ptr, &it->version)) {
+      Py_DECREF(pairs);
       Py_DECREF(w);
       return NULL;
     }
   }
+  Py_DECREF(pairs);
   return (PyObject*)w;
 }
 

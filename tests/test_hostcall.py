@@ -4,6 +4,7 @@ stand in for the compiled ones, CPU tensors for the device's."""
 import contextlib
 import copy
 import pickle
+import weakref
 
 import numpy as np
 import pytest
@@ -184,3 +185,27 @@ def test_replaced_structure_takes_the_full_path(which):
     args = kept_op_call(stub)
     args[which].add_(0)
     assert addmm_inplace._repeat(*args) is False and stub.calls == 0
+
+
+def test_watch_keeps_what_it_reads():
+    """A buffer's own methods may drop it from the dict that is being watched."""
+
+    class Buffer:
+        _version = 3
+
+        def __init__(self, buffers):
+            self.buffers = buffers
+
+        def data_ptr(self):
+            self.buffers.pop("a", None)
+            self.buffers["c"] = None
+            return 64
+
+    buffers = {}
+    buffers["a"], buffers["b"] = Buffer(buffers), Buffer(buffers)
+    last = weakref.ref(buffers["a"])
+    watch = _lib.hostcall().Watch(buffers)
+    assert last() is None and not watch.unchanged(buffers)
+    assert _lib.hostcall().Watch({"b": buffers["b"]}).unchanged({"b": buffers["b"]})
+    with pytest.raises(AttributeError):
+        _lib.hostcall().Watch({"a": 1})
