@@ -107,6 +107,11 @@ typedef enum {
   SSL_DEBUG_TOPK_GROUPS = 5
 } ssl_debug_knob;
 int ssl_debug_set(int32_t knob, int64_t value);
+/* What the calling thread's last ssl_slr_forward_group or ssl_bsr_addmm_inplace
+ * call launched: token rows per row tile (256, 128 or 64; 0 if it streamed or
+ * launched nothing) and the parts its row groups ran in (2 to 4; 1: whole; 0:
+ * by the members' part tables). */
+int ssl_debug_prefill_choice(int32_t* tile, int32_t* parts);
 
 /* Device bounds checks (no reference counterpart): 1 in the library's checked
  * build (compiled with SSL_DEVICE_CHECKS=1, libssalaad_amd_checked.so), 0 in

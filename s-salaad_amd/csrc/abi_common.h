@@ -35,4 +35,12 @@ struct DebugKnobs {
 };
 DebugKnobs& debug_knobs();
 
+// What the thread's last fused or in-place call ran (ssl_debug_prefill_choice):
+// token rows per tile (0: it streamed) and K parts (1: whole row groups, 0: the
+// part table).
+struct PrefillChoice {
+  int tile, parts;
+};
+PrefillChoice& prefill_choice();
+
 }  // namespace ssl

@@ -557,6 +557,7 @@ int ssl_bsr_addmm_inplace(void* out, int64_t ldo, const void* x, int64_t ldx, co
                           int32_t* counters, int64_t n_counters, void* workspace,
                           int64_t workspace_bytes, void* stream) {
   clear_error();
+  prefill_choice() = {};
   if (!supported_dtype(dtype)) return fail(SSL_ERR_UNSUPPORTED, "unsupported dtype %d", dtype);
   if (!supported_block(block_p, block_q))
     return fail(SSL_ERR_UNSUPPORTED,
@@ -617,7 +618,7 @@ int ssl_bsr_addmm_inplace(void* out, int64_t ldo, const void* x, int64_t ldx, co
         prefill_group_steps(nnz, n_chunks, K, block_p, pf_group, ssl_prefill_step_cols(dtype)), 0,
         device_cus(), rows.bm, dtype);
     const int64_t part_bytes = pm.ksplit * pf_n_groups * T * rows.bm * 64 * 4;
-    if (n_counters < ssl_bsr_addmm_counter_count(M, NB) || pf_n_groups > NB ||
+    if (n_counters < ssl_bsr_addmm_counter_count(M, NB) || pf_n_groups > NB || !workspace ||
         part_bytes > workspace_bytes - need || part_bytes > 0x7fffffffLL)
       pm.ksplit = 1;
     if (pm.ksplit > 1) {
@@ -626,6 +627,7 @@ int ssl_bsr_addmm_inplace(void* out, int64_t ldo, const void* x, int64_t ldx, co
     }
     rows.items = (int)(pf_n_groups * T * pm.ksplit);
     rows.off[1] = rows.items;
+    prefill_choice() = {rows.bm, pm.ksplit};
     return check_hip(prefill_launch_op(dtype, block_p, pf_group, rows, (hipStream_t)stream),
                      "bsr_addmm prefill launch");
   }
@@ -677,6 +679,7 @@ int ssl_slr_forward_group(const void* x, int64_t ldx, int64_t M, int64_t m, int6
                           int32_t block_p, int32_t block_q, int32_t dtype,
                           const ssl_slr_member* members, int32_t n_members, void* stream) {
   clear_error();
+  prefill_choice() = {};
   if (!supported_dtype(dtype)) return fail(SSL_ERR_UNSUPPORTED, "unsupported dtype %d", dtype);
   if (!supported_block(block_p, block_q))
     return fail(SSL_ERR_UNSUPPORTED,
@@ -915,6 +918,7 @@ int ssl_slr_forward_group(const void* x, int64_t ldx, int64_t M, int64_t m, int6
     lat.off[n_members] = (int)litems;
     rows.items = (int)items;
     lat.items = (int)litems;
+    prefill_choice() = {rows.bm, parts ? 0 : ksplit};
     if (nm)
       return check_hip(prefill_launch_fused_nm24(dtype, rows, lat, (hipStream_t)stream),
                        "slr prefill launch (2:4)");

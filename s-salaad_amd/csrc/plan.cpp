@@ -35,8 +35,10 @@ constexpr int64_t kMaxParts = 16;
 
 static thread_local std::string g_last_error;
 static DebugKnobs g_knobs{};
+static thread_local PrefillChoice g_choice{};
 
 DebugKnobs& debug_knobs() { return g_knobs; }
+PrefillChoice& prefill_choice() { return g_choice; }
 
 int fail(int code, const char* fmt, ...) {
   char buf[512];
@@ -117,6 +119,14 @@ int ssl_debug_set(int32_t knob, int64_t value) {
       return SSL_OK;
   }
   return fail(SSL_ERR_INVALID, "unknown debug knob %d", knob);
+}
+
+int ssl_debug_prefill_choice(int32_t* tile, int32_t* parts) {
+  clear_error();
+  if (!tile || !parts) return fail(SSL_ERR_INVALID, "null pointer");
+  *tile = prefill_choice().tile;
+  *parts = prefill_choice().parts;
+  return SSL_OK;
 }
 
 int ssl_plan_build(const int32_t* crow_host, const int32_t* col_host, int64_t NB, int64_t NBK,

@@ -57,6 +57,7 @@ _SIGNATURES = {
     ),
     "ssl_bsr_addmm_workspace_size": (_c_i64, [_c_i64, _c_i64, _c_i32, _c_i64]),
     "ssl_bsr_addmm_counter_count": (_c_i64, [_c_i64, _c_i64]),
+    "ssl_debug_prefill_choice": (ctypes.c_int, [_c_p, _c_p]),
     "ssl_bsr_addmm_inplace": (
         ctypes.c_int,
         [_c_p, _c_i64, _c_p, _c_i64, _c_p, _c_p, _c_i64, _c_p, _c_i64, _c_i64, _c_p, _c_p, _c_p,
@@ -279,6 +280,14 @@ def dtype_code(dtype: torch.dtype) -> int:
     if code is None:
         raise TypeError(f"SLR kernels support float32/bfloat16/float16, got {dtype}")
     return code
+
+
+def prefill_choice() -> tuple[int, int]:
+    """(row tile, K parts) of this thread's last call (ssl_debug_prefill_choice)."""
+    tile, parts = ctypes.c_int32(), ctypes.c_int32()
+    check(load().ssl_debug_prefill_choice(ctypes.byref(tile), ctypes.byref(parts)),
+          "ssl_debug_prefill_choice")
+    return tile.value, parts.value
 
 
 def check(rc: int, what: str) -> None:

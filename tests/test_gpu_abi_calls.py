@@ -85,6 +85,63 @@ def test_member_without_low_rank_factor(dtype, p, M, prefill, gpu_device):
     assert _runtime.read_status(gpu_device) == 0
 
 
+def _op_call(prob, x, out, counters, workspace, workspace_bytes):
+    """One ssl_bsr_addmm_inplace call of `prob`'s S with the scratch given."""
+    lib = _lib.load()
+    dev, dt, p = x.device, _lib.SSL_BF16, prob["p"]
+    crow, col, vt, act = orc.module_buffers(prob["crow"], prob["col"], prob["vals"])
+    M, NB, NBK = x.shape[0], prob["NB"], prob["NBK"]
+    table, n_chunks, n_slots = _runtime.build_plan(crow, col, NBK, act, p, 0, 0)
+    G = int(lib.ssl_prefill_group(M, n_chunks, p, p))
+    groups, steps, ng = _runtime.build_prefill_plan(crow, col, NBK, act, p, G, 64)
+    assert lib.ssl_bsr_addmm_takes_prefill(M, n_chunks, p, p, dt)
+    t = [torch.from_numpy(a).to(dev) for a in (table, col, groups, steps)]
+    vals = to_dev(vt, x.dtype, dev)
+    vpq = vals.transpose(1, 2).contiguous()
+    rc = lib.ssl_bsr_addmm_inplace(
+        out.data_ptr(), out.stride(0), x.data_ptr(), x.stride(0), t[1].data_ptr(), vals.data_ptr(),
+        vals.shape[0], t[0].data_ptr(), n_chunks, n_slots, vpq.data_ptr(), t[2].data_ptr(),
+        t[3].data_ptr(), ng, G, M, NB * p, NBK * p, NB, p, p, dt, counters.data_ptr(),
+        counters.numel(), _lib.ptr(workspace), workspace_bytes, _lib.stream_ptr(dev))
+    _lib.check(rc, "ssl_bsr_addmm_inplace")
+    torch.cuda.synchronize()
+    return _lib.prefill_choice()
+
+
+@pytest.mark.parametrize("scratch", ["full", "counters", "workspace", "none", "null"])
+def test_op_with_less_scratch_runs_whole_groups(scratch, gpu_device):
+    """A call that would run its groups in parts, given exactly the queries'
+    sizes, the streaming kernel's counters or workspace only, or a null
+    workspace that claims a size: the parts need both, everything else runs
+    whole groups with the same sums to fp32 rounding."""
+    lib = _lib.load()
+    dtype, M = torch.bfloat16, 300
+    prob = make_problem(2048, 5472, 64, 32, 0.5, dtype, seed=3)
+    crow, col, vt, act = orc.module_buffers(prob["crow"], prob["col"], prob["vals"])
+    x_np = make_x(prob, M, seed=5)
+    out0 = torch.from_numpy(np.random.default_rng(1).standard_normal((M, 2048))).to(dtype)
+    want = orc.bsr_addmm_inplace(out0.double().numpy(), x_np, crow, col, vt, act)
+    NB = prob["NB"]
+    n_cnt = int(lib.ssl_bsr_addmm_counter_count(M, NB))
+    n_min = -(-M // 64) * NB  # one per (64-row token tile, block-row)
+    nbytes = int(lib.ssl_bsr_addmm_workspace_size(M, NB, 32, 0))
+    assert n_min < n_cnt and nbytes > 0
+    counters = torch.zeros(n_min if scratch in ("counters", "none") else n_cnt, dtype=torch.int32,
+                           device=gpu_device)
+    ws = None
+    if scratch != "null":
+        size = 256 if scratch in ("workspace", "none") else nbytes
+        ws = torch.empty(size, dtype=torch.uint8, device=gpu_device)
+    out = out0.to(gpu_device)
+    print(f"[op scratch] {scratch}", flush=True)
+    tile, parts = _op_call(prob, to_dev(x_np, dtype, gpu_device), out, counters, ws,
+                           nbytes if ws is None else ws.numel())
+    assert parts > 1 if scratch == "full" else parts == 1
+    assert tile in (64, 128)
+    assert err(out, want) <= TOL[dtype]
+    assert int(counters.abs().max()) == 0
+
+
 @pytest.mark.parametrize("M,prefill", [(16, False), (256, True)])
 def test_nm24_member_without_low_rank_factor(M, prefill, gpu_device):
     dtype = torch.bfloat16
