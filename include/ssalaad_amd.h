@@ -254,7 +254,8 @@ int32_t ssl_bsr_addmm_takes_prefill(int64_t M, int64_t n_rows, int32_t block_p,
                                     int32_t block_q, int32_t dtype);
 /* The sizes include what a prefill call's K parts take; a call given less (at
  * least the streaming kernel's counters and partial tiles of split rows) runs
- * whole row groups. */
+ * whole row groups. The workspace for NB = 0 is what a call that streams
+ * (ssl_bsr_addmm_takes_prefill is 0) needs. */
 int64_t ssl_bsr_addmm_workspace_size(int64_t M, int64_t NB, int32_t block_p,
                                      int64_t n_slots);
 int64_t ssl_bsr_addmm_counter_count(int64_t M, int64_t NB);

@@ -150,6 +150,15 @@ int64_t op_workspace_min(int64_t M, int32_t block_p, int64_t n_slots) {
   const int64_t MG = (M + 16 * MT - 1) / (16 * MT);
   return align_up(4 * MG * n_slots * (16 * MT * block_p), 256);
 }
+// Arrival words of the parts: one per (token tile, group) of a grid that splits.
+// The library's own splits keep two parts or more of every group resident, three
+// workgroups a compute unit at most (prefill_row_split), so they are few; a
+// forced split (test hook) has one per (64-row tile, block-row) at most.
+int64_t op_arrivals(int64_t M, int64_t NB) {
+  if (M < kPrefillMinM) return 0;
+  const int64_t all = (M + 63) / 64 * NB, most = 3 * (int64_t)device_cus() / 2;
+  return debug_knobs().prefill_split != 0 || all < most ? all : most;
+}
 int64_t op_split_bytes(int64_t M, int64_t NB, int32_t block_p) {
   if (M < kPrefillMinM || !prefill_block(block_p, block_p, SSL_BF16)) return 0;
   return prefill_split_bytes(M, NB, block_p, 0, 0, SSL_BF16, device_cus());
@@ -536,10 +545,10 @@ int32_t ssl_bsr_addmm_takes_prefill(int64_t M, int64_t n_rows, int32_t block_p, 
   return 1;
 }
 
-// Row counters, then (many token rows) one arrival word per (64-row token
-// tile, block-row) for the tiled kernel's K parts, all zero at rest.
+// Row counters, then (many token rows) the arrival words of the tiled kernel's K
+// parts, all zero at rest.
 int64_t ssl_bsr_addmm_counter_count(int64_t M, int64_t NB) {
-  return op_counters_min(M, NB) + (M >= kPrefillMinM ? (M + 63) / 64 * NB : 0);
+  return op_counters_min(M, NB) + op_arrivals(M, NB);
 }
 
 // The streaming kernel's partial tiles of split rows, then (many token rows)
@@ -618,7 +627,7 @@ int ssl_bsr_addmm_inplace(void* out, int64_t ldo, const void* x, int64_t ldx, co
         prefill_group_steps(nnz, n_chunks, K, block_p, pf_group, ssl_prefill_step_cols(dtype)), 0,
         device_cus(), rows.bm, dtype);
     const int64_t part_bytes = pm.ksplit * pf_n_groups * T * rows.bm * 64 * 4;
-    if (n_counters < ssl_bsr_addmm_counter_count(M, NB) || pf_n_groups > NB || !workspace ||
+    if (n_counters < op_counters_min(M, NB) + pf_n_groups * T || !workspace ||
         part_bytes > workspace_bytes - need || part_bytes > 0x7fffffffLL)
       pm.ksplit = 1;
     if (pm.ksplit > 1) {

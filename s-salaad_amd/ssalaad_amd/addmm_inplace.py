@@ -299,7 +299,9 @@ def bsr_addmm_inplace_(
     dev = out_inplace.device
     with torch.cuda.device(dev):
         generation = _runtime.generation()
-        ws = _runtime.workspace(dev, lib.ssl_bsr_addmm_workspace_size(M, NB, block_p, plan.n_slots))
+        # a call that streams has no parts to keep tiles for
+        ws = _runtime.workspace(dev, lib.ssl_bsr_addmm_workspace_size(M, NB if pf else 0, block_p,
+                                                                      plan.n_slots))
         cnt = _runtime.counters(dev, lib.ssl_bsr_addmm_counter_count(M, NB))
         vals_pq = _values_pq(values, vals) if pf else None
         # built before the launch: nothing after it may raise for want of it

@@ -342,6 +342,20 @@ def test_workspace_sizes_are_aligned_and_monotone():
     assert lib.ssl_bsr_addmm_counter_count(65, 172) == 2 * 172
     assert lib.ssl_bsr_addmm_workspace_size(16, 172, 64, 0) == 0
     assert lib.ssl_bsr_addmm_workspace_size(16, 172, 64, 10) == 10 * 16 * 64 * 4
+    # from 128 rows (the tiled kernel) the op's parts too: their arrival words, of
+    # at most one and a half groups a compute unit (256 without a device), and
+    # their tiles (up to 4 parts of 64-row tiles, 128 × 64 fp32 each); none where
+    # even the tall grid fills the device, nor for calls that stream (NB = 0)
+    assert lib.ssl_bsr_addmm_counter_count(127, 172) == 2 * 172
+    assert lib.ssl_bsr_addmm_counter_count(128, 172) == 2 * 172 + 2 * 172
+    assert lib.ssl_bsr_addmm_counter_count(300, 172) == 5 * 172 + 384
+    assert lib.ssl_bsr_addmm_counter_count(2048, 688) == 32 * 688 + 384
+    assert lib.ssl_bsr_addmm_workspace_size(127, 64, 32, 0) == 0
+    assert lib.ssl_bsr_addmm_workspace_size(300, 64, 32, 0) == 4 * 5 * 32 * 128 * 64 * 4
+    assert lib.ssl_bsr_addmm_workspace_size(300, 172, 64, 0) == 4 * 256 * 128 * 64 * 4
+    assert lib.ssl_bsr_addmm_workspace_size(8192, 172, 64, 0) == 0
+    assert lib.ssl_bsr_addmm_workspace_size(300, 0, 32, 0) == 0
+    assert lib.ssl_bsr_addmm_workspace_size(300, 0, 64, 10) == 5 * 10 * 64 * 64 * 4
 
 
 def test_entry_points_reject_bad_arguments_before_any_launch():

@@ -200,6 +200,21 @@ def test_first_op_call_under_capture_allocates_no_pinned_memory(gpu_device, monk
     assert torch.equal(out, want)
 
 
+def test_streaming_op_calls_reserve_no_part_tiles(gpu_device, monkeypatch):
+    """fp32 calls of any token count stream: they ask for no room for the tiled
+    kernel's parts; a 16-bit call of the same size does."""
+    asked = []
+    real = _runtime.workspace
+    monkeypatch.setattr(_runtime, "workspace", lambda dev, n: (asked.append(n), real(dev, n))[1])
+    for dtype in (torch.float32, torch.bfloat16):
+        mod, _ = _linear(7, dtype=dtype, bias=False)
+        x, out = (torch.zeros(300, n, device="cuda", dtype=dtype) for n in (160, 192))
+        torch.ops.ssalaad.tilelang_bsr_addmm_inplace_dense_(out, x, mod.S_crow, mod.S_col,
+                                                            mod.S_values, mod.S_active_rows)
+        assert (_lib.prefill_choice()[0] > 0) == (dtype == torch.bfloat16)
+    assert asked[0] == 0 and asked[1] == _lib.load().ssl_bsr_addmm_workspace_size(300, 6, 32, 0) > 0
+
+
 def test_launchers_check_their_arguments():
     h = _lib.hostcall()
     with pytest.raises(ValueError):
