@@ -4,6 +4,7 @@
 
 #include <string.h>
 
+#include <algorithm>
 #include <vector>
 
 #include "abi_internal.h"
@@ -227,6 +228,12 @@ int check_member(int i, const ssl_slr_member& mb, int64_t M, int64_t m_pad, int 
   if (!aligned(mb.exchange, 256))
     return fail(SSL_ERR_WORKSPACE, "linear %d: exchange area must be 256-byte aligned", i);
   return SSL_OK;
+}
+
+// Whether the member has a part table and the workspace for its partial tiles.
+bool has_part_table(const ssl_slr_member& mb, const Layout& L, int64_t M) {
+  return mb.pf_parts && mb.pf_n_parts > 0 &&
+         mb.workspace_bytes >= L.total + ssl_prefill_parts_bytes(M, mb.pf_split_parts);
 }
 
 // The streaming kernel's arguments for one member (a latent split of n_kc
@@ -773,8 +780,35 @@ int ssl_slr_forward_group(const void* x, int64_t ldx, int64_t M, int64_t m, int6
     int ksplit = prefill_row_split(n_grp * ((M + rows.bm - 1) / rows.bm), grp_steps, lat_split, cus,
                                    rows.bm, dtype);
     const int64_t short_items = n_grp * ((M + 63) / 64);
-    if (rows.bm == 64 && short_items >= cus && dtype != SSL_F32 && knobs.prefill_split == 0 &&
-        knobs.prefill_group == 0) {
+    const bool free_tile = knobs.prefill_split == 0 && knobs.prefill_group == 0;
+    int kn = 1;  // the narrow tile's parts, where they compete with the short one's
+    if (rows.bm == 64 && short_items >= cus && dtype != SSL_F32 && free_tile)
+      kn = prefill_row_split(n_grp * ((M + 127) / 128), grp_steps, lat_split, cus, 128, dtype);
+    // Skewed structures: equal parts of every group leave the longest group's k
+    // times shorter at best, the part table cuts it to about the mean. So the
+    // tables run (below, groups otherwise whole) when their long groups fall into
+    // more parts than k on average: 4096×11008 with Zipf 64×64 blocks at 40% (22
+    // long groups of 64, 2.5 parts each) at 384 rows 59 µs by the table, 82 in two
+    // equal parts; 1184×9088 with 32×32 at 24% (2.8) at 256 30 in four, 34 by the
+    // table. They count their own workgroups for the short tile, up to two and a
+    // quarter a unit: that Zipf shape short / narrow at 256 rows (392 parts) 48 / 52,
+    // at 384 (588) 66 / 59; 4064×4480 with 32×32 at 18% at 346 (516) 28 / 32.
+    int64_t long_groups = 0, long_parts = 0, table_parts = 0;
+    bool tables = knobs.prefill_split == 0 && knobs.prefill_group != 2 &&
+                  n_grp * ((M + 255) / 256) <= 4 * (int64_t)cus;
+    for (int i = 0; i < n_members && tables; ++i) {
+      const ssl_slr_member& mb = members[i];
+      if (mb.NB == 0) continue;
+      tables = has_part_table(mb, L[i], M);
+      table_parts += mb.pf_n_parts;
+      long_parts += mb.pf_split_parts;
+      long_groups += mb.pf_n_groups - (mb.pf_n_parts - mb.pf_split_parts);
+    }
+    if (tables && long_groups > 0 && long_parts >= std::max(ksplit, kn) * long_groups) {
+      ksplit = 1;
+      if (rows.bm == 64 && free_tile && 4 * table_parts * ((M + 63) / 64) > 9 * (int64_t)cus)
+        rows.bm = 128;
+    } else if (kn > ksplit || (kn == ksplit && kn > 1 && block_p == 64)) {
       // from one short workgroup a compute unit on, more narrow parts are better,
       // and as many with 64×64 blocks, whose steps always load a whole weight
       // tile: 4096×11008 with 64×64 at 50% (86 steps) at 256 rows narrow in two
@@ -783,12 +817,8 @@ int ssl_slr_forward_group(const void* x, int64_t ldx, int64_t M, int64_t m, int6
       // narrow in 3 58.0, short in two 62.1; 2:4 2048×8192 (128) at 600 narrow in
       // 3 60.9, short whole 91.1. With fewer: 1600×8192 with 32×32 at 90% (127) at
       // 512 rows (200 short) narrow in 3 61.4, short in two 55.5.
-      const int kn = prefill_row_split(n_grp * ((M + 127) / 128), grp_steps, lat_split, cus, 128,
-                                       dtype);
-      if (kn > ksplit || (kn == ksplit && kn > 1 && block_p == 64)) {
-        rows.bm = 128;
-        ksplit = kn;
-      }
+      rows.bm = 128;
+      ksplit = kn;
     }
     for (int i = 0; i < n_members && ksplit > 1; ++i) {
       const ssl_slr_member& mb = members[i];
@@ -829,9 +859,7 @@ int ssl_slr_forward_group(const void* x, int64_t ldx, int64_t M, int64_t m, int6
         if (members[i].NB > 0) tall += members[i].pf_n_groups * ((M + 255) / 256);
       for (int i = 0; i < n_members && tall <= 4 * (int64_t)cus; ++i) {
         const ssl_slr_member& mb = members[i];
-        if (mb.NB > 0 && mb.pf_parts && mb.pf_n_parts > 0 &&
-            mb.workspace_bytes >= L[i].total + ssl_prefill_parts_bytes(M, mb.pf_split_parts))
-          parts = true;
+        if (mb.NB > 0 && has_part_table(mb, L[i], M)) parts = true;
       }
       if (parts && rows.bm == 256) rows.bm = 128;
     }
@@ -848,8 +876,7 @@ int ssl_slr_forward_group(const void* x, int64_t ldx, int64_t M, int64_t m, int6
         const ssl_slr_member& mb = members[i];
         if (mb.NB == 0) continue;
         const int64_t T = (M + rows.bm - 1) / rows.bm;
-        const bool mp = parts && mb.pf_parts && mb.pf_n_parts > 0 &&
-                        mb.workspace_bytes >= L[i].total + ssl_prefill_parts_bytes(M, mb.pf_split_parts);
+        const bool mp = parts && has_part_table(mb, L[i], M);
         row_items += (mp ? mb.pf_n_parts : mb.pf_n_groups) * T;
         if (mb.r_pad > 0) lat_items += TL * (mb.r_pad / 64);
       }
@@ -907,8 +934,7 @@ int ssl_slr_forward_group(const void* x, int64_t ldx, int64_t M, int64_t m, int6
       lat.mb[i].ksplit = ls.split;
       lat.mb[i].kchunk = ls.chunk;
       lat.mb[i].kpart = (float*)((char*)mb.workspace + L[i].pf_split + rows_bytes);
-      if (parts && mb.pf_parts && mb.pf_n_parts > 0 &&
-          mb.workspace_bytes >= L[i].total + ssl_prefill_parts_bytes(M, mb.pf_split_parts)) {
+      if (parts && has_part_table(mb, L[i], M)) {
         if (mb.pf_n_parts < mb.pf_n_groups || mb.pf_split_parts < 0 ||
             mb.pf_split_parts > mb.pf_n_parts || mb.pf_n_parts > 0x7fffffffLL / 8)
           return fail(SSL_ERR_INVALID, "linear %d: part table sizes do not fit its plan", i);

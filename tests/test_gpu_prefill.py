@@ -18,7 +18,7 @@ import pytest
 import torch
 
 from oracle import slr_oracle as orc
-from slr_cases import TOL, err, make_module, make_problem, make_x, oracle_y, to_dev
+from slr_cases import TOL, err, make_module, make_nm_module, make_problem, make_x, oracle_y, to_dev
 
 import ssalaad_amd
 from ssalaad_amd import _lib
@@ -283,6 +283,43 @@ def test_tile_and_parts_of_small_grids(n, m, p, dtype, M, gpu_device):
     torch.cuda.synchronize()
     assert err(y, oracle_y(prob, x)) <= TOL[dtype]
     assert _counters_at_rest(gpu_device)
+
+
+@pytest.mark.parametrize("kind,n,m,p,density,skew,M,choice", [
+    # skewed: the part table where its long groups fall into more parts than k
+    ("linear", 2048, 11008, 64, 0.3, True, 256, (64, 0)),
+    ("linear", 2048, 8192, 32, 0.2, True, 256, (64, 0)),
+    ("linear", 1184, 9088, 32, 0.24, True, 256, (64, 3)),
+], ids=lambda v: str(v).replace(" ", "") if not isinstance(v, bool) else ("skew" if v else "even"))
+def test_choice_of_tile_and_parts(kind, n, m, p, density, skew, M, choice, gpu_device):
+    """The row tile and K parts (0: the part table) that a call runs on a device
+    of 256 compute units, on either side of the rules that pick them, and the
+    call's result."""
+    dtype, dev = torch.bfloat16, gpu_device
+    if torch.cuda.get_device_properties(dev).multi_processor_count != 256:
+        pytest.skip("the rules' lines are stated for 256 compute units")
+    if kind == "nm":
+        mod, (A, B, S, b) = make_nm_module(n, m, 128, dtype, dev, seed=M)
+        x = torch.from_numpy(np.random.default_rng(M).standard_normal((M, m))).to(dtype)
+        y = mod(x.to(dev))
+        assert _lib.prefill_choice() == choice
+        want = orc.slr_linear(x.double().numpy(), A, B, S, b)
+    else:
+        prob = make_problem(n, m, 128, p, density, dtype, seed=n + M, skew=skew)
+        x = make_x(prob, M, seed=M)
+        if kind == "linear":
+            y = make_module(prob, dev)(to_dev(x, dtype, dev))
+            want = oracle_y(prob, x)
+        else:
+            crow, col, vt, act = orc.module_buffers(prob["crow"], prob["col"], prob["vals"])
+            y = torch.zeros(M, n, dtype=dtype, device=dev)
+            torch.ops.ssalaad.tilelang_bsr_addmm_inplace_dense_(
+                y, to_dev(x, dtype, dev), torch.from_numpy(crow).to(dev),
+                torch.from_numpy(col).to(dev), to_dev(vt, dtype, dev), torch.from_numpy(act).to(dev))
+            want = orc.bsr_addmm_inplace(np.zeros((M, n)), x, crow, col, vt, act)
+        assert _lib.prefill_choice() == choice
+    assert err(y, want) <= TOL[dtype]
+    assert _counters_at_rest(dev)
 
 
 # -------------------------------------------- full size, library's choice --
