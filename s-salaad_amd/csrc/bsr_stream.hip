@@ -624,15 +624,22 @@ int ssl_bsr_addmm_inplace(void* out, int64_t ldo, const void* x, int64_t ldx, co
     pm.values_bytes = nnz * block_p * block_q * eb;
     pm.groups = pf_groups; pm.steps = pf_steps; pm.n_groups = (int)pf_n_groups;
     rows.bm = prefill_row_tile(M, n_chunks, pf_group, block_p, device_cus(), dtype, 0);
-    const int64_t T = (M + rows.bm - 1) / rows.bm;
-    if (pf_n_groups * T > 0x7fffffffLL / 8) return fail(SSL_ERR_INVALID, "grid too large");
     // K parts when the row grid is small (prefill_row_split) and the counters
     // and workspace hold their arrivals and partial tiles (a call with less
     // runs whole groups)
-    pm.ksplit = prefill_row_split(
-        pf_n_groups * T,
-        prefill_group_steps(nnz, n_chunks, K, block_p, pf_group, ssl_prefill_step_cols(dtype)), 0,
-        device_cus(), rows.bm, dtype);
+    const int step_cols = ssl_prefill_step_cols(dtype);
+    const int64_t steps = prefill_group_steps(nnz, n_chunks, K, block_p, pf_group, step_cols);
+    int64_t T;
+    for (;;) {
+      T = (M + rows.bm - 1) / rows.bm;
+      if (pf_n_groups * T > 0x7fffffffLL / 8) return fail(SSL_ERR_INVALID, "grid too large");
+      pm.ksplit = prefill_row_split(pf_n_groups * T, steps, 0, device_cus(), rows.bm, dtype);
+      if (rows.bm != 64 || pm.ksplit > 1 ||
+          !prefill_narrow_over_short(M, pf_n_groups, steps, K / step_cols, block_p, device_cus(),
+                                     dtype))
+        break;
+      rows.bm = 128;
+    }
     const int64_t part_bytes = pm.ksplit * pf_n_groups * T * rows.bm * 64 * 4;
     if (n_counters < op_counters_min(M, NB) + pf_n_groups * T || !workspace ||
         part_bytes > workspace_bytes - need || part_bytes > 0x7fffffffLL)
@@ -817,6 +824,11 @@ int ssl_slr_forward_group(const void* x, int64_t ldx, int64_t M, int64_t m, int6
       // narrow in 3 58.0, short in two 62.1; 2:4 2048×8192 (128) at 600 narrow in
       // 3 60.9, short whole 91.1. With fewer: 1600×8192 with 32×32 at 90% (127) at
       // 512 rows (200 short) narrow in 3 61.4, short in two 55.5.
+      rows.bm = 128;
+      ksplit = kn;
+    } else if (rows.bm == 64 && ksplit == 1 && !nm &&
+               prefill_narrow_over_short(M, n_grp, grp_steps, m_pad / step_cols, block_p, cus,
+                                         dtype)) {
       rows.bm = 128;
       ksplit = kn;
     }

@@ -126,6 +126,10 @@ int prefill_group(int64_t M, int64_t n_rows, int block_p, int n_cus);
 // lat_items: the latent's workgroups in the same launch.
 int prefill_row_tile(int64_t M, int64_t n_rows, int group, int block_p, int n_cus, int dtype,
                      int64_t lat_items);
+// Whether whole groups (no K parts) of a grid that the short tile was chosen for
+// run on the narrow one after all. all_steps: a group's steps were it full.
+bool prefill_narrow_over_short(int64_t M, int64_t groups, int64_t steps, int64_t all_steps,
+                               int block_p, int n_cus, int dtype);
 // Whether `tall` workgroups of the tall tile (2 a compute unit) finish before
 // `narrow` workgroups of the narrow one (3 a compute unit, the latent's
 // included); false while a test forces the tile.

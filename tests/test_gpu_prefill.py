@@ -290,6 +290,13 @@ def test_tile_and_parts_of_small_grids(n, m, p, dtype, M, gpu_device):
     ("linear", 2048, 11008, 64, 0.3, True, 256, (64, 0)),
     ("linear", 2048, 8192, 32, 0.2, True, 256, (64, 0)),
     ("linear", 1184, 9088, 32, 0.24, True, 256, (64, 3)),
+    # whole groups past one short workgroup a unit: narrow where they are many,
+    # long and mostly full
+    ("linear", 5888, 2432, 16, 0.3, False, 151, (128, 1)),
+    ("op", 5888, 2432, 16, 0.3, False, 151, (128, 1)),
+    ("op", 5472, 2048, 32, 0.5, False, 129, (128, 1)),
+    ("op", 5472, 2048, 32, 0.3, False, 192, (64, 1)),
+    ("linear", 4096, 2048, 64, 0.5, False, 300, (64, 1)),
 ], ids=lambda v: str(v).replace(" ", "") if not isinstance(v, bool) else ("skew" if v else "even"))
 def test_choice_of_tile_and_parts(kind, n, m, p, density, skew, M, choice, gpu_device):
     """The row tile and K parts (0: the part table) that a call runs on a device
