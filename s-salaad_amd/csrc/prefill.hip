@@ -39,6 +39,8 @@
 // by every XCD at about the same time, so the 256 MB MALL serves all but the
 // first read).
 
+#include <algorithm>
+
 #include "abi_internal.h"
 #include "prefill.h"
 #include "slr_common.h"
@@ -1081,6 +1083,12 @@ hipError_t launch_fused(const PfArgs& rows, const PfArgs& lat, int P, int G, hip
 // steps a group) at 256 rows 17.7 / 19.8 / 21.1 / 25.9; 1024×4096 (48) 25.2 /
 // 18.5 / 18.7 / 21.1; 2048×5461 (64) 49.6 / 38.3 / 33.9 / 38.4.
 constexpr int64_t kRowSplitMinSteps = 20;
+// Up to half a workgroup a compute unit 16-bit parts pay from 16 steps on, in up
+// to three: 752×2176 with 16×16 blocks (34 steps, 36 short workgroups) at 155 rows
+// 18.9 whole, 15.8 in two; 768×3072 with 16×16 at 85% (48, 60) at 300 23.2 in two,
+// 19.8 in three; 1600×8192 with 32×32 at 30% (65, 100) at 256 27.0 in three, 29.1 in
+// four.
+constexpr int64_t kRowSplitFewSteps = 16, kRowSplitFewMost = 3;
 // Short 16-bit tiles from one workgroup per compute unit on share a unit's load
 // path and their parts have to be longer: 4096×11008 with 64×64 blocks at 30%
 // (52 steps) at 256 rows (256 workgroups) 39.9 whole, 42.9 in two parts;
@@ -1114,6 +1122,8 @@ int prefill_row_split(int64_t items, int64_t steps, int64_t lat_items, int n_cus
   int64_t k = steps / (narrow ? kRowSplitNarrowSteps
                        : dtype != SSL_F32 && items >= n_cus ? kRowSplitLongSteps
                                                             : kRowSplitMinSteps);
+  if (!narrow && 2 * items <= n_cus && dtype != SSL_F32)
+    k = std::max(k, std::min(steps / kRowSplitFewSteps, kRowSplitFewMost));
   // (three parts of 256 groups: the op's 4096×11008 at 256 rows 41.2 µs in two,
   // 45.0; four of 128 groups: 2048×8192 at 200 rows with 16×16 at 30% (97 steps)
   // 32.5 in three, 33.5, and 2:4 (128) 40.4 in three, 37.9)

@@ -297,6 +297,10 @@ def test_tile_and_parts_of_small_grids(n, m, p, dtype, M, gpu_device):
     ("op", 5472, 2048, 32, 0.5, False, 129, (128, 1)),
     ("op", 5472, 2048, 32, 0.3, False, 192, (64, 1)),
     ("linear", 4096, 2048, 64, 0.5, False, 300, (64, 1)),
+    # at most half a workgroup a unit: two or three parts from 16 steps each
+    ("linear", 768, 2176, 16, 0.83, False, 155, (64, 2)),
+    ("op", 768, 3072, 16, 0.85, False, 300, (64, 3)),
+    ("linear", 2048, 2048, 32, 0.5, False, 256, (64, 1)),
 ], ids=lambda v: str(v).replace(" ", "") if not isinstance(v, bool) else ("skew" if v else "even"))
 def test_choice_of_tile_and_parts(kind, n, m, p, density, skew, M, choice, gpu_device):
     """The row tile and K parts (0: the part table) that a call runs on a device
