@@ -785,12 +785,12 @@ int ssl_slr_forward_group(const void* x, int64_t ldx, int64_t M, int64_t m, int6
     }
     if (n_grp > 0) grp_steps /= n_grp;
     int ksplit = prefill_row_split(n_grp * ((M + rows.bm - 1) / rows.bm), grp_steps, lat_split, cus,
-                                   rows.bm, dtype);
+                                   rows.bm, dtype, nm);
     const int64_t short_items = n_grp * ((M + 63) / 64);
     const bool free_tile = knobs.prefill_split == 0 && knobs.prefill_group == 0;
     int kn = 1;  // the narrow tile's parts, where they compete with the short one's
     if (rows.bm == 64 && short_items >= cus && dtype != SSL_F32 && free_tile)
-      kn = prefill_row_split(n_grp * ((M + 127) / 128), grp_steps, lat_split, cus, 128, dtype);
+      kn = prefill_row_split(n_grp * ((M + 127) / 128), grp_steps, lat_split, cus, 128, dtype, nm);
     // Skewed structures: equal parts of every group leave the longest group's k
     // times shorter at best, the part table cuts it to about the mean. So the
     // tables run (below, groups otherwise whole) when their long groups fall into

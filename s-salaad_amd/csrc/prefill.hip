@@ -1100,6 +1100,10 @@ constexpr int64_t kRowSplitLongSteps = 28;
 // whole, 66.2 in two parts; the op's 4096×11008 with 64×64 (86) at 512 rows 60.4 /
 // 54.6; 3200×8640 with 32×32 (101) at 384 rows 68.3 / 63.6, in 3 parts 58.0.
 constexpr int64_t kRowSplitNarrowSteps = 33;
+// 2:4 steps run on the structured-sparse MFMA and load 5/8 of the weight bytes, so
+// a round of them costs less: 4096×4096 (64 steps) at 340 / 512 rows short whole
+// 49.6 / 52.1, narrow in two 44.5 / 48.3.
+constexpr int64_t kRowSplitNarrowStepsNm = 28;
 
 int64_t prefill_group_steps(int64_t nnz, int64_t rows, int64_t m_pad, int block_p, int group,
                             int step_cols) {
@@ -1112,14 +1116,14 @@ int64_t prefill_group_steps(int64_t nnz, int64_t rows, int64_t m_pad, int block_
 }
 
 int prefill_row_split(int64_t items, int64_t steps, int64_t lat_items, int n_cus, int bm,
-                      int dtype) {
+                      int dtype, bool nm) {
   if (bm >= 256) return 1;  // the tall tile keeps its registers for its own steps
   const int64_t forced = debug_knobs().prefill_split;  // test hook
   if (forced == 1) return 1;
   if (forced >= 2) return (int)forced;
   if (items <= 0) return 1;
   const bool narrow = bm > 64;
-  int64_t k = steps / (narrow ? kRowSplitNarrowSteps
+  int64_t k = steps / (narrow ? (nm ? kRowSplitNarrowStepsNm : kRowSplitNarrowSteps)
                        : dtype != SSL_F32 && items >= n_cus ? kRowSplitLongSteps
                                                             : kRowSplitMinSteps);
   if (!narrow && 2 * items <= n_cus && dtype != SSL_F32)

@@ -301,6 +301,9 @@ def test_tile_and_parts_of_small_grids(n, m, p, dtype, M, gpu_device):
     ("linear", 768, 2176, 16, 0.83, False, 155, (64, 2)),
     ("op", 768, 3072, 16, 0.85, False, 300, (64, 3)),
     ("linear", 2048, 2048, 32, 0.5, False, 256, (64, 1)),
+    # 2:4: narrow parts from 28 steps
+    ("nm", 4096, 4096, 32, 0.5, False, 340, (128, 2)),
+    ("nm", 4096, 3072, 32, 0.5, False, 340, (64, 1)),
 ], ids=lambda v: str(v).replace(" ", "") if not isinstance(v, bool) else ("skew" if v else "even"))
 def test_choice_of_tile_and_parts(kind, n, m, p, density, skew, M, choice, gpu_device):
     """The row tile and K parts (0: the part table) that a call runs on a device
