@@ -2,10 +2,12 @@
 one, and whatever differs from it — weights, shapes, strides, streams, a refused
 status — takes the full path again with the full path's results and errors."""
 
+from concurrent.futures import ThreadPoolExecutor
+
 import pytest
 import torch
 
-from ssalaad_amd import LRSLinear, LRSLinearGroup, _lib, _runtime, clear_wait_status, prepare_bsr_addmm
+from ssalaad_amd import LRSLinear, LRSLinearGroup, _lib, _runtime, addmm_inplace, clear_wait_status, prepare_bsr_addmm
 
 pytestmark = pytest.mark.gpu
 
@@ -54,18 +56,61 @@ def test_repeated_linear_calls(n, m, tokens, gpu_device):
     assert mod(x[:0]).shape == (0, n)
 
 
+class Counting:
+    """A kept launcher that counts the calls issued through it."""
+
+    def __init__(self, launcher):
+        self.launcher, self.calls = launcher, 0
+
+    def launch(self, *args):
+        self.calls += 1
+        return self.launcher.launch(*args)
+
+
+def _live(kept, call):
+    """Repeat `call` until its launcher is in the dict that `kept()` returns;
+    then count what goes through it, one call among others."""
+    for _ in range(4):
+        call()
+        if kept():
+            break
+    (key, entry), = list(kept().items())
+    at, = [i for i, v in enumerate(entry) if type(v).__name__ in ("GroupCall", "OpCall")]
+    counting = Counting(entry[at])
+    kept()[key] = entry[:at] + (counting,) + entry[at + 1:]
+    call()
+    assert counting.calls == 1
+    return counting
+
+
+def _replace_b(mod):
+    mod.B = mod.B * 3
+
+
+def _new_bias_storage(mod):
+    mod.bias.data = mod.bias * 0 + 1
+
+
+def _drop_bias(mod):
+    mod.bias = None
+
+
+@pytest.mark.parametrize("change", [lambda mod: mod.A.mul_(2), _replace_b, _new_bias_storage,
+                                    _drop_bias, lambda mod: mod.S_values.mul_(1)],
+                         ids=["in-place", "replaced", "new-storage", "dropped", "S-in-place"])
+def test_changed_weights_leave_the_launcher(change, gpu_device):
+    mod, S = _linear(1)
+    x = torch.randn(4, 160, device="cuda").to(torch.bfloat16)
+    counting = _live(lambda: mod._state._launchers, lambda: mod(x))
+    change(mod)
+    _close(mod(x), _expect(mod, S, x))
+    assert counting.calls == 1
+
+
 def test_changed_weights_and_refusals(gpu_device):
     mod, S = _linear(1)
     x = torch.randn(4, 160, device="cuda").to(torch.bfloat16)
-    mod(x), mod(x)
-    mod.A.mul_(2)                       # in place
-    _close(mod(x), _expect(mod, S, x))
-    mod.B = mod.B * 3                   # replaced
-    _close(mod(x), _expect(mod, S, x))
-    mod.bias.data = mod.bias * 0 + 1    # new storage, same tensor object
-    _close(mod(x), _expect(mod, S, x))
-    mod.bias = None
-    _close(mod(x), _expect(mod, S, x))
+    counting = _live(lambda: mod._state._launchers, lambda: mod(x))
     with pytest.raises(TypeError):
         mod(x.half())
     with pytest.raises(ValueError):
@@ -74,14 +119,34 @@ def test_changed_weights_and_refusals(gpu_device):
         mod(x.cpu())
     word = _runtime.status_word(x.device)
     word._word.value = 1
+    assert counting.launcher.launch(x.data_ptr(), x.data_ptr()) == -1  # nothing is launched
     try:
         with pytest.raises(RuntimeError):
             mod(x)
     finally:
         clear_wait_status()
+    assert counting.calls == 2  # the refused call asked it, and no other did
     _close(mod(x), _expect(mod, S, x))
+    assert counting.calls == 3
     mod.half()
     _close(mod(x.half()), _expect(mod, S, x.half()))
+    assert counting.calls == 3
+
+
+def test_threads_share_a_launcher(gpu_device):
+    """Each call fills in a copy of the descriptors: threads that use one module
+    (on one stream, so that its scratch is ordered) get their own outputs."""
+    mod, S = _linear(8)
+    xs = [torch.randn(4, 160, device="cuda").to(torch.bfloat16) for _ in range(4)]
+    want = [mod(x) for x in xs]
+    counting = _live(lambda: mod._state._launchers, lambda: mod(xs[0]))
+    torch.cuda.synchronize()
+    with ThreadPoolExecutor(4) as pool:
+        got = list(pool.map(lambda x: [mod(x) for _ in range(50)], xs))
+    torch.cuda.synchronize()
+    assert counting.calls == 201
+    for ys, w in zip(got, want):
+        assert all(torch.equal(y, w) for y in ys)
 
 
 def test_groups_streams_and_grown_pools(gpu_device):
@@ -90,9 +155,18 @@ def test_groups_streams_and_grown_pools(gpu_device):
     grp = LRSLinearGroup(a, b)
     x = torch.randn(3, 160, device="cuda").to(torch.bfloat16)
     first = [y.clone() for y in grp(x)]
+    counting = _live(lambda: a._state._launchers, lambda: grp(x))
     for y, (mod, S) in zip(first, ((a, Sa), (b, Sb))):
         _close(y, _expect(mod, S, x))
     assert all(torch.equal(u, v) for u, v in zip(grp(x), first))
+    assert counting.calls == 2
+    word = _runtime.status_word(x.device)
+    word._word.value = 1
+    assert counting.launcher.launch(*[x.data_ptr()] * 3) == -1
+    with pytest.raises(RuntimeError):
+        grp(x)
+    word.clear()
+    calls = counting.calls
     side = torch.cuda.Stream()
     side.wait_stream(torch.cuda.current_stream())
     with torch.cuda.stream(side):
@@ -101,14 +175,17 @@ def test_groups_streams_and_grown_pools(gpu_device):
     side.synchronize()
     before = _runtime.generation()
     big = torch.randn(400, 160, device="cuda").to(torch.bfloat16)
-    for u, v in zip(grp(big[:3]), grp(big)):
-        assert u.shape[0] == 3 and v.shape[0] == 400
+    _close(grp(big)[0], _expect(a, Sa, big))
     _runtime.workspace(x.device, _runtime.workspace(x.device, 1).numel() + 1)  # a grown pool
     assert _runtime.generation() > before
     for _ in range(2):
         assert all(torch.equal(u, v) for u, v in zip(grp(x), first))
+    assert counting.calls == calls  # bound to the first stream and the outgrown pool
+    a._state._launchers.clear()
+    counting = _live(lambda: a._state._launchers, lambda: grp(x))
     b.A.add_(1)
     _close(grp(x)[1], _expect(b, Sb, x))
+    assert counting.calls == 1
 
 
 @pytest.mark.parametrize("tokens", [1, 7, 100])
@@ -126,6 +203,9 @@ def test_repeated_op_calls(tokens, gpu_device):
         return out_
 
     first = run(x, out0, vals)
+    kept = lambda: getattr(crow, addmm_inplace._PLAN_ATTR).calls  # noqa: E731
+    assert _lib.prefill_choice() == (0, 0)
+    counting = _live(kept, lambda: run(x, out0, vals))
     _close(first, out0.double() + x.double() @ S.double().T)
     for _ in range(2):
         assert torch.equal(run(x, out0, vals), first)
@@ -133,11 +213,32 @@ def test_repeated_op_calls(tokens, gpu_device):
     vals.mul_(0.5)
     _close(run(x, out0, vals), out0.double() + 0.5 * (x.double() @ S.double().T))
     vals.mul_(2)
+    assert counting.calls == 5  # other values too: they are read anew
     wide = torch.empty(tokens, 168, device="cuda", dtype=x.dtype)
     wide[:, 1:161] = x
     assert torch.equal(run(wide[:, 1:161], out0, vals), first)
     with pytest.raises(TypeError):
         run(x.half(), out0, vals)
+    assert counting.calls == 5
+    counting = _live(kept, lambda: run(x, out0, vals))
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        for _ in range(3):
+            assert torch.equal(run(x, out0, vals), first)
+    side.synchronize()
+    assert counting.calls == 1 and len(kept()) == 2
+    word = _runtime.status_word(x.device)
+    word._word.value = 1
+    assert counting.launcher.launch(*[x.data_ptr()] * 3) == -1
+    with pytest.raises(RuntimeError):
+        run(x, out0, vals)
+    word.clear()
+    calls = counting.calls
+    _runtime.workspace(x.device, _runtime.workspace(x.device, 1).numel() + 1)  # a grown pool
+    for _ in range(3):
+        assert torch.equal(run(x, out0, vals), first)
+    assert counting.calls == calls
     act2 = act[:-1].clone()  # fewer active rows: the last block-row keeps its bits
     out = out0.clone()
     op(out, x, crow, col, vals, act2)

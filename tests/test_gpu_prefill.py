@@ -263,23 +263,27 @@ def test_op_in_k_parts(dtype, p, mode, k, tile, split, gpu_device):
         outs = [to_dev(out0, dtype, dev) for _ in range(2)]
         for out in outs:
             torch.ops.ssalaad.tilelang_bsr_addmm_inplace_dense_(out, to_dev(x, dtype, dev), *args)
+            assert _lib.prefill_choice() == (64 if mode == SHORT else 128, k)
         assert _counters_at_rest(dev), M
         assert err(outs[0], want) <= TOL[dtype], M
         assert torch.equal(outs[0], outs[1]), M
 
 
-@pytest.mark.parametrize("n,m,p,dtype,M", [
-    (1024, 4096, 32, torch.bfloat16, 200),   # 64 short workgroups, in parts
-    (4096, 11008, 64, torch.bfloat16, 256),  # 256 of them: narrow, in parts
-    (1024, 2048, 32, torch.float32, 1024),   # fp32, in two parts
-    (4096, 4096, 64, torch.bfloat16, 384),   # 384 of them: short, whole
+@pytest.mark.parametrize("n,m,p,dtype,M,choice", [
+    (1024, 4096, 32, torch.bfloat16, 200, (64, 3)),   # 64 short workgroups, in parts
+    (4096, 11008, 64, torch.bfloat16, 256, (128, 2)),  # 256 of them: narrow, in parts
+    (1024, 2048, 32, torch.float32, 1024, (64, 2)),   # fp32, in two parts
+    (4096, 4096, 64, torch.bfloat16, 384, (64, 1)),   # 384 of them: short, whole
 ], ids=["short-parts", "narrow-parts", "f32-parts", "short-whole"])
-def test_tile_and_parts_of_small_grids(n, m, p, dtype, M, gpu_device):
-    """The library's own choice of tile and parts on either side of its rules."""
+def test_tile_and_parts_of_small_grids(n, m, p, dtype, M, choice, gpu_device):
+    """The library's own choice of tile and parts (on 256 compute units) on
+    either side of its rules."""
     prob = make_problem(n, m, 128, p, 0.5, dtype, seed=n + M)
     mod = make_module(prob, gpu_device)
     x = make_x(prob, M, seed=M)
     y = mod(to_dev(x, dtype, gpu_device))
+    if torch.cuda.get_device_properties(gpu_device).multi_processor_count == 256:
+        assert _lib.prefill_choice() == choice
     torch.cuda.synchronize()
     assert err(y, oracle_y(prob, x)) <= TOL[dtype]
     assert _counters_at_rest(gpu_device)
