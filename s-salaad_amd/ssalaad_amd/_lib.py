@@ -229,13 +229,16 @@ def load() -> ctypes.CDLL:
 _hostcall = None
 
 
-def hostcall():
-    """The compiled host call path (once); raises if it was not built."""
+def hostcall(required: bool = True):
+    """The compiled host call path (once); raises if it was not built (None then
+    unless `required`)."""
     global _hostcall
     if _hostcall is None:
         try:
             from . import hostcall as mod
         except ImportError as e:
+            if not required:
+                return None
             raise RuntimeError(
                 "the host call path is not built; run `python s-salaad_amd/build.py` "
                 "(or __graft_entry__.build()) first") from e

@@ -51,7 +51,7 @@ def get_tuned_config(block_p: int, block_q: int) -> dict:
 
 
 class _StructPlan:
-    __slots__ = ("versions", "col_ref", "act_ref", "plans", "NB_K", "calls")
+    __slots__ = ("versions", "col_ref", "act_ref", "plans", "NB_K", "calls", "seen", "tiled")
 
     def __init__(self, versions, col, act, NB_K):
         self.versions = versions
@@ -59,8 +59,11 @@ class _StructPlan:
         self.act_ref = weakref.ref(act)
         self.plans: dict[int, _runtime.DevicePlan] = {}
         self.NB_K = NB_K
-        # streaming calls already made: (shapes, stream) -> (generation, launcher)
+        # streaming calls made twice: (shapes, stream) -> (generation, launcher),
+        # and those made once
         self.calls: dict[tuple, tuple] = {}
+        self.seen: set[tuple] = set()
+        self.tiled: set[int] = set()  # token counts whose calls have no launcher
 
 
 _PLAN_ATTR = "_ssl_struct_plan"
@@ -92,15 +95,15 @@ def _validated_host_structure(crow, col, active_rows, nnz_values, NB_K):
     return crow_h.astype(np.int32), act_h.astype(np.int32)
 
 
-def _versions(crow, col, active_rows) -> tuple:
+def _versions(crow, col, active_rows, nnz, NB_K) -> tuple:
     """What a structure's plans and launchers were built from."""
     return (crow._version, col._version, active_rows._version, crow.data_ptr(), col.data_ptr(),
-            active_rows.data_ptr())
+            active_rows.data_ptr(), nnz, NB_K)
 
 
 def _plan_for(crow, col, active_rows, values, NB_K, block_p, block_q, M, elem_bytes,
               prefill=None):
-    versions = _versions(crow, col, active_rows) + (values.shape[0], NB_K)
+    versions = _versions(crow, col, active_rows, values.shape[0], NB_K)
     sp = getattr(crow, _PLAN_ATTR, None)
     if (
         sp is None
@@ -127,6 +130,9 @@ def _plan_for(crow, col, active_rows, values, NB_K, block_p, block_q, M, elem_by
     if prefill is None:
         prefill = bool(lib.ssl_bsr_addmm_takes_prefill(M, plan.n_chunks, block_p, block_q, dt))
     if prefill and plan.n_chunks > 0:
+        if len(sp.tiled) >= _MAX_TILED:
+            sp.tiled.clear()
+        sp.tiled.add(M)
         # the prefill kernel's groups list the planned rows (active rows with blocks)
         G = int(lib.ssl_prefill_group(M, plan.n_chunks, block_p, block_q))
         step_cols = int(lib.ssl_prefill_step_cols(dt))
@@ -188,7 +194,11 @@ def _aligned_rows(t: torch.Tensor) -> bool:
     return t.stride(-1) == 1 and t.data_ptr() % 16 == 0 and (t.stride(0) * eb) % 16 == 0
 
 
-_MAX_CALLS = 16  # kept launchers per structure
+# Kept launchers per structure: one per token count of a decode batch. Calls of
+# more counts in turn keep finding their count new and build none (building one
+# for every call and dropping it took 2.4 of 16.9 µs).
+_MAX_CALLS = 64
+_MAX_TILED = 4096
 
 
 def _repeat(out, x, crow, col, values, active) -> bool:
@@ -196,7 +206,8 @@ def _repeat(out, x, crow, col, values, active) -> bool:
     shapes on its stream, with contiguous 16-byte aligned tensors; False when
     it is not one (or would be refused): the full path then handles it."""
     sp = getattr(crow, _PLAN_ATTR, None)
-    if sp is None or sp.col_ref() is not col or sp.act_ref() is not active:
+    if (sp is None or not sp.calls or x.dim() != 2 or x.shape[0] in sp.tiled
+            or sp.col_ref() is not col or sp.act_ref() is not active):
         return False
     dev = crow.device
     if torch._C._cuda_getDevice() != dev.index:
@@ -208,11 +219,25 @@ def _repeat(out, x, crow, col, values, active) -> bool:
     if (out.dtype is not values.dtype or x.dtype is not values.dtype or out.device != dev
             or x.device != dev or values.device != dev
             or not (out.is_contiguous() and x.is_contiguous() and values.is_contiguous())
-            or sp.versions[:-2] != _versions(crow, col, active)):
+            or sp.versions != _versions(crow, col, active, *sp.versions[-2:])):
         return False
     o, xp, v = out.data_ptr(), x.data_ptr(), values.data_ptr()
     return (o | xp | v) % 16 == 0 and _lib.issued(hit[1].launch(o, xp, v),
                                                   "ssl_bsr_addmm_inplace")
+
+
+def _keeps(sp: _StructPlan, key: tuple) -> bool:
+    """Whether the call of this key gets a launcher: its second one, or one
+    whose launcher is bound to replaced buffers."""
+    hit = sp.calls.get(key)
+    if hit is not None:
+        return hit[0] != _runtime.generation()
+    if key in sp.seen:
+        return True
+    if len(sp.seen) >= _MAX_CALLS:
+        sp.seen.clear()
+    sp.seen.add(key)
+    return False
 
 
 def bsr_addmm_inplace_(
@@ -304,11 +329,16 @@ def bsr_addmm_inplace_(
                                                                       plan.n_slots))
         cnt = _runtime.counters(dev, lib.ssl_bsr_addmm_counter_count(M, NB))
         vals_pq = _values_pq(values, vals) if pf else None
-        # built before the launch: nothing after it may raise for want of it
+        # built before the launch: nothing after it may raise; the op itself does
+        # without the host call path
         launcher = None
         if (pf is None and target is out_inplace and out_inplace.is_contiguous()
-                and x.is_contiguous() and col is col_indices and dev.index is not None):
-            launcher = _lib.hostcall().OpCall(
+                and x.is_contiguous() and col is col_indices and dev.index is not None
+                and _keeps(sp := getattr(crow_indices, _PLAN_ATTR),
+                           key := (out_inplace.shape, x.shape, values.shape, values.dtype,
+                                   _lib.stream_ptr(dev)))
+                and (host := _lib.hostcall(required=False)) is not None):
+            launcher = host.OpCall(
                 _lib.entry_address("ssl_bsr_addmm_inplace"), _runtime.status_address(dev),
                 N, K, col.data_ptr(), vals.shape[0], plan.table.data_ptr(), plan.n_chunks,
                 plan.n_slots, M, N, K, NB, block_p, block_q, dt, cnt.data_ptr(), cnt.numel(),
@@ -324,11 +354,9 @@ def bsr_addmm_inplace_(
         )
     _lib.check(rc, "ssl_bsr_addmm_inplace")
     if launcher is not None:
-        calls = getattr(crow_indices, _PLAN_ATTR).calls
-        if len(calls) >= _MAX_CALLS:
-            calls.clear()
-        calls[(out_inplace.shape, x.shape, values.shape, values.dtype, _lib.stream_ptr(dev))] = (
-            generation, launcher)
+        if len(sp.calls) >= _MAX_CALLS:
+            sp.calls.clear()
+        sp.calls[key] = (generation, launcher)
     if target is not out_inplace:
         out_inplace.copy_(target)
 

@@ -2,6 +2,7 @@
 one, and whatever differs from it — weights, shapes, strides, streams, a refused
 status — takes the full path again with the full path's results and errors."""
 
+import sys
 from concurrent.futures import ThreadPoolExecutor
 
 import pytest
@@ -133,6 +134,20 @@ def test_changed_weights_and_refusals(gpu_device):
     assert counting.calls == 3
 
 
+def test_a_kept_launcher_is_not_built_again(gpu_device, monkeypatch):
+    """Calls that cannot use it (an x that is copied first) leave it as it is."""
+    mod, S = _linear(9)
+    x = torch.randn(4, 160, device="cuda").to(torch.bfloat16)
+    wide = torch.empty(4, 184, device="cuda", dtype=x.dtype)
+    wide[:, 3:163] = x
+    counting = _live(lambda: mod._state._launchers, lambda: mod(x))
+    monkeypatch.setattr(_lib, "hostcall", lambda **kw: pytest.fail("built again"))
+    for _ in range(3):
+        _close(mod(wide[:, 3:163]), _expect(mod, S, x))
+    mod(x)
+    assert counting.calls == 2
+
+
 def test_threads_share_a_launcher(gpu_device):
     """Each call fills in a copy of the descriptors: threads that use one module
     (on one stream, so that its scratch is ordered) get their own outputs."""
@@ -220,14 +235,13 @@ def test_repeated_op_calls(tokens, gpu_device):
     with pytest.raises(TypeError):
         run(x.half(), out0, vals)
     assert counting.calls == 5
-    counting = _live(kept, lambda: run(x, out0, vals))
     side = torch.cuda.Stream()
     side.wait_stream(torch.cuda.current_stream())
     with torch.cuda.stream(side):
         for _ in range(3):
             assert torch.equal(run(x, out0, vals), first)
     side.synchronize()
-    assert counting.calls == 1 and len(kept()) == 2
+    assert counting.calls == 5 and len(kept()) == 2
     word = _runtime.status_word(x.device)
     word._word.value = 1
     assert counting.launcher.launch(*[x.data_ptr()] * 3) == -1
@@ -245,23 +259,23 @@ def test_repeated_op_calls(tokens, gpu_device):
     assert torch.equal(out[:, -32:], out0[:, -32:]) and torch.equal(out[:, :-32], first[:, :-32])
 
 
-def test_op_without_the_host_call_path_leaves_out_as_it_was(gpu_device, monkeypatch):
-    """A missing extension is found before the launch: out keeps its bits, so a
-    call made again after the error adds x·Sᵀ once."""
-    mod, _ = _linear(5, bias=False)
+def test_op_does_without_the_host_call_path(gpu_device, monkeypatch):
+    """Where the extension is not built every call of the op takes the full path;
+    none raises after the kernel has added to out."""
+    mod, S = _linear(5, bias=False)
     args = [t.clone() for t in (mod.S_crow, mod.S_col, mod.S_values, mod.S_active_rows)]
     x = torch.randn(3, 160, device="cuda").to(torch.bfloat16)
-    out = torch.randn(3, 192, device="cuda").to(torch.bfloat16)
-    before = out.clone()
-
-    def missing():
-        raise RuntimeError("the host call path is not built")
-
-    monkeypatch.setattr(_lib, "hostcall", missing)
+    out0 = torch.randn(3, 192, device="cuda").to(torch.bfloat16)
+    monkeypatch.setattr(_lib, "_hostcall", None)
+    monkeypatch.setitem(sys.modules, "ssalaad_amd.hostcall", None)  # its import fails
+    monkeypatch.delattr("ssalaad_amd.hostcall")
     with pytest.raises(RuntimeError, match="not built"):
+        _lib.hostcall()
+    for _ in range(4):
+        out = out0.clone()
         torch.ops.ssalaad.tilelang_bsr_addmm_inplace_dense_(out, x, *args)
-    torch.cuda.synchronize()
-    assert torch.equal(out, before)
+        _close(out, out0.double() + x.double() @ S.double().T)
+    assert not getattr(args[0], addmm_inplace._PLAN_ATTR).calls
 
 
 def test_first_op_call_under_capture_allocates_no_pinned_memory(gpu_device, monkeypatch):

@@ -39,7 +39,7 @@ def kept_op_call(stub, nb=2, p=16):
     act = torch.arange(nb, dtype=torch.int32)
     vals = torch.zeros(nb, p, p)
     out, x = torch.zeros(3, nb * p), torch.zeros(3, p)
-    sp = addmm_inplace._StructPlan(addmm_inplace._versions(crow, col, act) + (nb, 1), col, act, 1)
+    sp = addmm_inplace._StructPlan(addmm_inplace._versions(crow, col, act, nb, 1), col, act, 1)
     sp.calls[(out.shape, x.shape, vals.shape, vals.dtype, 0)] = (_runtime.generation(), stub)
     setattr(crow, addmm_inplace._PLAN_ATTR, sp)
     return out, x, crow, col, vals, act
@@ -209,3 +209,38 @@ def test_watch_keeps_what_it_reads():
     assert _lib.hostcall().Watch({"b": buffers["b"]}).unchanged({"b": buffers["b"]})
     with pytest.raises(AttributeError):
         _lib.hostcall().Watch({"a": 1})
+
+
+def test_op_builds_a_launcher_for_repeated_calls_only(monkeypatch):
+    """A call's second time builds its launcher, a replaced buffer builds it
+    anew, and more token counts in turn than are kept build none at all."""
+    crow = torch.zeros(2, dtype=torch.int32)
+    sp = addmm_inplace._StructPlan((), crow, crow, 1)
+    most = addmm_inplace._MAX_CALLS
+    assert not any(addmm_inplace._keeps(sp, (M,)) for M in range(most))
+    assert all(addmm_inplace._keeps(sp, (M,)) for M in range(most))
+    sp.calls[(1,)] = (_runtime.generation(), Stub())
+    assert not addmm_inplace._keeps(sp, (1,))
+    _runtime._replaced()
+    assert addmm_inplace._keeps(sp, (1,))
+    sp = addmm_inplace._StructPlan((), crow, crow, 1)
+    assert not any(addmm_inplace._keeps(sp, (M,)) for M in list(range(most + 1)) * 3)
+
+
+def test_op_calls_without_a_launcher_are_left_at_once():
+    """Tiled token counts (no launcher is kept for them) and an x that is to be
+    refused for its dimensions."""
+    stub = Stub()
+    out, x, *rest = kept_op_call(stub)
+    assert addmm_inplace._repeat(out, x[0], *rest) is False
+    assert addmm_inplace._repeat(out, x[0, 0], *rest) is False
+    getattr(rest[0], addmm_inplace._PLAN_ATTR).tiled.add(3)
+    assert addmm_inplace._repeat(out, x, *rest) is False and stub.calls == 0
+
+
+def test_full_path_of_unchanged_weights_reads_the_buffers_once(monkeypatch):
+    mod, x = kept_linear(Stub(_lib.SSL_ERR_INVALID))
+    grp, gx = kept_group(Stub(_lib.SSL_ERR_INVALID))
+    monkeypatch.setattr(ls_linear, "_launch", lambda states, x, outf: [x] * len(states))
+    monkeypatch.setattr(ls_linear._LRSLinearBase, "_weights_key", lambda mod: pytest.fail("again"))
+    assert mod(x) is x and grp(gx) == (gx, gx)
