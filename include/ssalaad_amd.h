@@ -90,7 +90,8 @@ int ssl_status_word_alloc(void** host_ptr, void** device_ptr);
  *                               in_features) across workgroups; 1: never; 2
  *                               to 4: every such call splits its row groups in
  *                               that many parts (when the caller's workspace
- *                               holds the partial tiles).
+ *                               and counters hold the partial tiles and their
+ *                               arrivals).
  *   SSL_DEBUG_CHAIN_FRAG        0: the library decides whether a chained launch
  *                               of 32- or 64-wide blocks passes its stages'
  *                               inputs in fragment order (ssl_slr_stage.xf);

@@ -500,9 +500,12 @@ int32_t ssl_slr_takes_prefill(int64_t M, int64_t n_rows, int32_t block_p, int32_
   }
   if (debug_knobs().prefill_group != 0) return 1;  // a forced row tile (test hook)
   // The streaming kernel keeps only one-token-tile calls with at most 2048
-  // output features: its finer K split wins there (2048×2048 and 2048×5461
-  // with 32×32 blocks at 128 rows: 26.9 / 39.4 µs streaming against 28.8 /
-  // 42.0). Everywhere else the tiled kernels, K parts included, win: 16×16
+  // output features, a line drawn when the tiled kernels ran them in whole groups.
+  // With parts it holds where a group is too short to split (µs at 128 rows,
+  // streaming / tiled: 2048×2048 with 32×32 blocks 17.4 / 18.2, 1024×1024 13.0 /
+  // 13.5, 1024×2048 with 16×16 17.2 / 19.3) and costs time where it is not (2048×5461
+  // with 32×32 25.2 / 22.1, 1024×4096 26.0 / 20.4, 2048×5461 with 16×16 38.5 / 24.5).
+  // Everywhere else the tiled kernels, K parts included, win: 16×16
   // blocks 2.2-4.3× (11008×4096 at 128 / 256 / 512 rows 109 / 196 / 372 ->
   // 49 / 60 / 87 µs), 4096×11008 with 32×32 or 64×64 at 128 rows 82 / 64 ->
   // 46 / 44, 4096×4096 with 64×64 at 128 rows 34.3 -> 31.0.
@@ -540,11 +543,13 @@ int32_t ssl_bsr_addmm_takes_prefill(int64_t M, int64_t n_rows, int32_t block_p, 
   if (debug_knobs().prefill_group != 0) return 1;
   if (dtype == SSL_F32) return 0;
   // One token tile whose grid of short (64-row) tiles would fill at most a
-  // quarter of the CUs streams: the op's tiled kernel runs whole row groups (2048×5461
-  // with 32×32 blocks at 128 rows: 22.8 µs streaming, 36.0 tiled; 4096×4096
-  // and 4096×11008 with 64×64: 31.3 / 50.3 against 34.2 / 54.1), while
-  // 11008×4096 with 64×64 (172 groups) and 16×16 blocks tile (36.4 against
-  // 53.3, 51.5 against 109.4).
+  // quarter of the CUs streams. The line is from when the op's tiled kernel ran
+  // whole row groups (2048×5461 with 32×32 blocks 36.0 µs then); in K parts it is
+  // as fast or faster there too (µs at 128 rows, streaming / tiled: 2048×2048 with
+  // 32×32 14.1 / 14.1, 2048×5461 18.5 / 16.3, 1024×4096 18.5 / 13.5; with 64×64
+  // 4096×4096 22.7 / 15.7, 4096×11008 45.0 / 27.3), so moving it would gain.
+  // 11008×4096 with 64×64 (172 groups) and 16×16 blocks tile (24.9 and, 2048×5461,
+  // 17.9).
   if (M <= kPrefillMinM && block_p >= 32) {
     const int64_t per = 64 / block_p, groups = (n_rows + per - 1) / per;
     if (4 * groups <= device_cus()) return 0;
@@ -934,7 +939,8 @@ int ssl_slr_forward_group(const void* x, int64_t ldx, int64_t M, int64_t m, int6
         ls = prefill_latent_split(M, m_pad, mb.r_pad, dtype);
       } else if (mb.r_pad > 0) {
         // whole row groups: the latent splits when it is longer than their
-        // sparse steps and the workspace holds its partial tiles
+        // sparse steps (counted per block-row, so an upper bound on the union that
+        // a group of small blocks walks) and the workspace holds its partial tiles
         const int64_t group_steps = mb.nnz * block_p / ssl_prefill_step_cols(dtype) /
                                     (mb.pf_n_groups > 0 ? mb.pf_n_groups : 1);
         ls = prefill_latent_split_whole(M, m_pad, mb.r_pad, dtype,
