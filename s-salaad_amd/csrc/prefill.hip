@@ -1259,18 +1259,20 @@ int prefill_row_tile(int64_t M, int64_t n_rows, int group, int block_p, int n_cu
 
 // Past one short workgroup a compute unit some units run two, which share a
 // unit's load path and each load the group's weights; where the groups are many
-// (wide outputs, so few token tiles), long (17 steps) and mostly full, one narrow workgroup
-// takes less. Short / narrow µs: the op's 7616×1344 with 16×16 blocks at 48% (119
-// groups, 19 of 21 steps) at 168 rows 18.4 / 15.4, 8000×1536 with 32×32 at 63% (125,
-// 21 of 24) at 183 19.8 / 17.3, the linear's 5904×2432 with 16×16 at 30% (93, 29 of
-// 38) at 151 26.1 / 24.4. Not so with 64×64 blocks (7424×832 at 50% at 187 8.9 /
-// 10.5), short groups (5472×2048 with 32×32 at 30%, 16 of 32 steps, at 192 14.3 /
-// 16.0) or few (768×3072 with 16×16 at 50%, 12 groups, at 1400 29.6 / 36.3).
+// (wide outputs, so few token tiles), 18 to 40 steps long and mostly full, one
+// narrow workgroup takes less. Short / narrow µs: the op's 7616×1344 with 16×16
+// blocks at 48% (119 groups, 19 of 21 steps) at 168 rows 18.4 / 15.4, 8000×1536 with
+// 32×32 at 63% (125, 21 of 24) at 183 19.8 / 17.3, the linear's 5904×2432 with 16×16
+// at 30% (93, 29 of 38) at 151 26.1 / 24.4. Not so with 64×64 blocks (7424×832 at 50%
+// at 187 8.9 / 10.5), longer groups, whose own steps hide the shared loads (5472×3072
+// with 16×16 at 82%, 48 steps, at 256: linear 36.2 / 39.6, op 34.6 / 36.9), short
+// ones (5472×2048 with 32×32 at 30%, 16 of 32 steps, at 192 14.3 / 16.0) or few
+// (768×3072 with 16×16 at 50%, 12 groups, at 1400 29.6 / 36.3).
 bool prefill_narrow_over_short(int64_t M, int64_t groups, int64_t steps, int64_t all_steps,
                                int block_p, int n_cus, int dtype) {
   if (debug_knobs().prefill_group != 0 || debug_knobs().prefill_split != 0) return false;
   return dtype != SSL_F32 && block_p < 64 && ((M + 63) / 64) * groups > n_cus && groups >= 40 &&
-         steps >= 17 && 2 * steps >= all_steps;
+         steps >= 18 && steps <= 40 && 2 * steps >= all_steps;
 }
 
 bool prefill_rounds_prefer_tall(int64_t tall, int64_t narrow, int n_cus) {

@@ -295,12 +295,13 @@ def test_tile_and_parts_of_small_grids(n, m, p, dtype, M, choice, gpu_device):
     ("linear", 2048, 8192, 32, 0.2, True, 256, (64, 0)),
     ("linear", 1184, 9088, 32, 0.24, True, 256, (64, 3)),
     # whole groups past one short workgroup a unit: narrow where they are many,
-    # long and mostly full
+    # of 18 to 40 steps and mostly full
     ("linear", 5888, 2432, 16, 0.3, False, 151, (128, 1)),
     ("op", 5888, 2432, 16, 0.3, False, 151, (128, 1)),
     ("op", 5472, 2048, 32, 0.5, False, 129, (128, 1)),
     ("op", 5472, 2048, 32, 0.3, False, 192, (64, 1)),
     ("linear", 4096, 2048, 64, 0.5, False, 300, (64, 1)),
+    ("linear", 5472, 3072, 16, 0.82, False, 256, (64, 1)),
     # at most half a workgroup a unit: two or three parts from 16 steps each
     ("linear", 768, 2176, 16, 0.83, False, 155, (64, 2)),
     ("op", 768, 3072, 16, 0.85, False, 300, (64, 3)),
