@@ -219,11 +219,14 @@ def _repeat(out, x, crow, col, values, active) -> bool:
     if (out.dtype is not values.dtype or x.dtype is not values.dtype or out.device != dev
             or x.device != dev or values.device != dev
             or not (out.is_contiguous() and x.is_contiguous() and values.is_contiguous())
-            or sp.versions != _versions(crow, col, active, *sp.versions[-2:])):
+            or sp.versions[:6] != (crow._version, col._version, active._version, crow.data_ptr(),
+                                   col.data_ptr(), active.data_ptr())):
         return False
     o, xp, v = out.data_ptr(), x.data_ptr(), values.data_ptr()
-    return (o | xp | v) % 16 == 0 and _lib.issued(hit[1].launch(o, xp, v),
-                                                  "ssl_bsr_addmm_inplace")
+    if (o | xp | v) % 16:
+        return False
+    rc = hit[1].launch(o, xp, v)
+    return rc == 0 or _lib.issued(rc, "ssl_bsr_addmm_inplace")
 
 
 def _keeps(sp: _StructPlan, key: tuple) -> bool:

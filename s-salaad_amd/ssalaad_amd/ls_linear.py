@@ -130,13 +130,6 @@ class _KernelState:
         self._pf_plans: dict[int, _runtime.DevicePrefillPlan] = {}
         self._values_pq: torch.Tensor | None = None
 
-    def views(self, mod: "_LRSLinearBase") -> bool:
-        """Whether mod.A still has this view's dtype and device: a reinterpreted
-        A keeps its pointer and version, and the calls it refuses are refused by
-        the full path."""
-        A = mod._buffers["A"]
-        return A.dtype is self.dtype and A.device == self.device
-
     def _padded(self, t: torch.Tensor, rows: int, cols: int) -> torch.Tensor:
         if t.shape == (rows, cols) and t.is_contiguous() and t.data_ptr() % 16 == 0:
             return t
@@ -390,11 +383,13 @@ def _relaunch(states, x: torch.Tensor, out_features):
     if len(pads) == 1:
         n, pad = out_features[0], pads[0]
         y = torch.empty((*lead, pad), dtype=x.dtype, device=x.device)
-        if not _lib.issued(launcher.launch(xp, y.data_ptr()), "ssl_slr_forward_group"):
+        rc = launcher.launch(xp, y.data_ptr())
+        if rc != 0 and not _lib.issued(rc, "ssl_slr_forward_group"):
             return None
         return (y if n == pad else y[..., :n],)
     ys = [torch.empty((*lead, pad), dtype=x.dtype, device=x.device) for pad in pads]
-    if not _lib.issued(launcher.launch(xp, *[y.data_ptr() for y in ys]), "ssl_slr_forward_group"):
+    rc = launcher.launch(xp, *[y.data_ptr() for y in ys])
+    if rc != 0 and not _lib.issued(rc, "ssl_slr_forward_group"):
         return None
     return [y if n == pad else y[..., :n] for y, n, pad in zip(ys, out_features, pads)]
 
@@ -537,9 +532,11 @@ class _LRSLinearBase(nn.Module):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         st = self._state
-        if (st is not None and st.watch.unchanged(self._buffers) and st.views(self)
-                and x.dtype is st.dtype and x.shape[-1] == self.in_features
-                and x.device == st.device):
+        # a reinterpreted A keeps its pointer and version: its dtype and device are
+        # compared too, and what they refuse is refused below
+        if (st is not None and st.watch.unchanged(self._buffers)
+                and x.dtype is (A := self._buffers["A"]).dtype is st.dtype
+                and x.shape[-1] == self.in_features and x.device == A.device == st.device):
             out = _relaunch((st,), x, (self.out_features,))
             return out[0] if out is not None else st.forward(x, self.out_features)
         if x.dtype != self.A.dtype:
@@ -757,7 +754,8 @@ class LRSLinearGroup(nn.Module):
         states, outf = [], []
         for mod in self.members._modules.values():
             st = mod._state
-            if st is None or not (st.watch.unchanged(mod._buffers) and st.views(mod)):
+            if (st is None or not st.watch.unchanged(mod._buffers)
+                    or (A := mod._buffers["A"]).dtype is not st.dtype or A.device != st.device):
                 return None
             states.append(st)
             outf.append(mod.out_features)
