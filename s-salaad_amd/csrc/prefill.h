@@ -94,15 +94,13 @@ constexpr int kPfLatArriveWord = 64;  // rank tiles ≤ 64 (r_pad ≤ 4096) for 
 int64_t prefill_group_steps(int64_t nnz, int64_t rows, int64_t m_pad, int block_p, int group,
                             int step_cols);
 // K parts of a prefill call with few row workgroups: each row group's sparse
-// steps (`steps` a group) in up to 4 parts of at least 20 steps (28 for
-// 16-bit calls from one workgroup per compute unit on, 33 for the narrow
-// tile, 28 for its 2:4 steps;
-// from 16 on in two or three for 16-bit calls of at most half a workgroup a unit),
-// as long as the parts are resident at once: with the latent's workgroups (`lat_items`, its K
-// chunks included) three a compute unit for the short tile, by themselves two
-// for the narrow one. The latent's in_features then split too
-// (prefill_latent_split), so neither leaves the other's critical path. 1 = no
-// split.
+// steps (`steps` a group) in up to 4 parts of at least 20 steps (28 for 16-bit
+// calls from one workgroup per compute unit on, 33 for the narrow tile, 28 for its
+// 2:4 steps; from 16 on in two or three for 16-bit calls of at most half a workgroup
+// a unit), as long as the parts are resident at once: with the latent's workgroups
+// (`lat_items`, its K chunks included) three a compute unit for the short tile, by
+// themselves two for the narrow one. The latent's in_features then split too
+// (prefill_latent_split), so neither leaves the other's critical path. 1 = no split.
 int prefill_row_split(int64_t items, int64_t steps, int64_t lat_items, int n_cus, int bm,
                       int dtype, bool nm = false);
 struct PfLatentSplit {
